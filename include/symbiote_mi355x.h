@@ -394,6 +394,10 @@ int sym_moe_down_fp8(const void* h, int T, int H, int I, const int32_t* seg_expe
  *   any number of stream-ordered launches (and graph replays). Launches that may overlap in time
  *   (on different streams) must use different workspaces. A smaller workspace returns
  *   SYM_ERR_WORKSPACE.
+ * sym_moe_gate_up_fp8_tiled / sym_moe_down_fp8_tiled: the same over fp8 e4m3fn expert weights with
+ *   128 x 128 block scales (layouts as sym_moe_gate_up_fp8 / sym_moe_down_fp8; y fp32): 128 x 256
+ *   tiles for segments of many rows. H % 256 == 0, I % 128 == 0, at most 512 segments; workspace as
+ *   above.
  */
 size_t sym_moe_tiled_workspace_bytes(void);
 int sym_gemm_bf16(const void* a, const void* w, const void* bias, const float* residual, int M,
@@ -405,6 +409,17 @@ int sym_moe_gate_up_tiled(const void* x, int T, int H, int I, int rows,
                           const int32_t* seg_offset, const int32_t* seg_count,
                           const int32_t* n_segments, int max_segments, const void* w_gate_up,
                           void* h, void* workspace, size_t workspace_bytes, void* stream);
+int sym_moe_gate_up_fp8_tiled(const void* x, int T, int H, int I, int rows,
+                              const int32_t* sorted_tokens, const int32_t* seg_expert,
+                              const int32_t* seg_offset, const int32_t* seg_count,
+                              const int32_t* n_segments, int max_segments, const void* w_gate_up,
+                              const float* s_gate_up, void* h, void* workspace,
+                              size_t workspace_bytes, void* stream);
+int sym_moe_down_fp8_tiled(const void* h, int T, int H, int I, int rows,
+                           const int32_t* seg_expert, const int32_t* seg_offset,
+                           const int32_t* seg_count, const int32_t* n_segments, int max_segments,
+                           const void* w_down, const float* s_down, float* y, void* workspace,
+                           size_t workspace_bytes, void* stream);
 int sym_moe_down_tiled(const void* h, int T, int H, int I, int rows, const int32_t* seg_expert,
                        const int32_t* seg_offset, const int32_t* seg_count,
                        const int32_t* n_segments, int max_segments, const void* w_down, void* y,

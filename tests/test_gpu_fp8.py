@@ -77,6 +77,50 @@ def test_grouped_swiglu_fp8(device, T, E, H, I, top_k, skew):
         torch.testing.assert_close(yk[rows], y_ref, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("T,E,H,I,top_k,hot", [
+    (1, 64, 512, 128, 4, 0),            # segments of one row; two steps of I
+    (37, 64, 512, 128, 2, 0),            # 16-row sub-tile remainders
+    (63, 64, 1024, 256, 4, 1),           # a thin tile one row short of full
+    (65, 64, 512, 384, 4, 1),            # one row past the thin tile: a 128-row tile
+    (300, 64, 1024, 256, 4, 2),         # 128-row tiles with thin remainders
+    (700, 256, 2048, 512, 8, 3),        # the model's shape, skewed
+    (40, 64, 8704, 128, 2, 0),           # more than 64 K-steps (scales reloaded)
+])
+def test_grouped_swiglu_fp8_tiled(device, monkeypatch, T, E, H, I, top_k, hot):
+    """The tiled fp8 kernels (forced for small T) against fp32 torch over the dequantised bytes,
+    as above; the streaming kernels agree to fp32 summation order."""
+    g = torch.Generator(device=device).manual_seed(T + H)
+    x = torch.randn(T, H, generator=g, device=device).bfloat16()
+    q = []
+    for shape in ((E + 1, 2 * I, H), (E + 1, H, I)):
+        q.append(hip_ops.quantize_block_fp8(
+            (torch.randn(shape, generator=g, device=device) * 0.05).bfloat16()))
+    logits = torch.randn(T, E, generator=g, device=device) * 2
+    logits[:, :hot] += 6.0
+    res = hip_ops.moe_route_permute(logits, torch.zeros(E, device=device), n_group=8,
+                                    topk_group=4, top_k=top_k, routed_scale=2.5,
+                                    with_shared=True)
+    hs, ys = hip_ops.moe_grouped_swiglu(x, res, *q, kernel="stream")
+    monkeypatch.setattr(hip_ops, "TILED_MIN_TOKENS_FP8", 1)
+    h = torch.full_like(hs, float("nan"))
+    y = torch.full_like(ys, float("nan"))
+    hip_ops.moe_grouped_swiglu(x, res, *q, h=h, y=y)
+    torch.cuda.synchronize()
+    wgu, wd = (w.q.float() * w.scale.repeat_interleave(128, -2).repeat_interleave(128, -1)
+               for w in q)
+    ns = int(res.n_segments.item())
+    for e, o, c in zip(res.seg_expert.cpu()[:ns].tolist(), res.seg_offset.cpu()[:ns].tolist(),
+                       res.seg_count.cpu()[:ns].tolist()):
+        xe = x[res.sorted_tokens[o:o + c].long()].float()
+        h_ref = F.silu(xe @ wgu[e, :I].T) * (xe @ wgu[e, I:].T)
+        # h: one bf16 rounding (2^-9) of an fp32 value
+        _close(h[o:o + c], h_ref, atol=2e-3, rtol=8e-3)
+        y_ref = h[o:o + c].float() @ wd[e].T
+        torch.testing.assert_close(y[o:o + c], y_ref, rtol=1e-4, atol=1e-4)
+    # the same products in another fp32 order; h may round to the neighbouring bf16 value
+    _close(h, hs, atol=2e-3, rtol=8e-3)
+
+
 # ------------------------------------------------------------------------------ KV fill
 def _fp8_pools(nb, Hkv, bs, device):
     """Empty fp8 pools: K [nb, Hkv, bs, 128], V dim-major [nb, Hkv, 128, bs], and scales."""

@@ -135,6 +135,16 @@ _SIGNATURES = {
         [_vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _vp, _vp, _vp,
          _c_size, _vp],
     ),
+    "sym_moe_gate_up_fp8_tiled": (
+        _c_int,
+        [_vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _vp,
+         _c_size, _vp],
+    ),
+    "sym_moe_down_fp8_tiled": (
+        _c_int,
+        [_vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _vp,
+         _c_size, _vp],
+    ),
     "sym_moe_down_tiled": (
         _c_int,
         [_vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _c_int, _vp, _vp, _c_int, _vp,

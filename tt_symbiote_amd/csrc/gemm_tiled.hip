@@ -73,7 +73,8 @@ struct TileArgs {
   long long out_zstride;    // ... and output plane out + z * out_zstride (elements)
   int full_rt;              // DENSE with tail_rows > 0: row tiles 0 .. full_rt - 1 have TM rows,
   int tail_rows;            // the rows from full_rt * TM on tiles of tail_rows (one plane)
-  int* tickets;             // gemm_tile_persistent: the caller's 8 per-XCD tile counters
+  int* tickets;             // persistent grids: the caller's 8 per-XCD tile counters
+  const float* w_scale;     // fp8 weights: [S, rows / 128, K / 128] block scales
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -856,20 +857,17 @@ constexpr size_t kTicketBytes = 8 * sizeof(int);
 // the fetch-add has a whole tile to return. Tickets 0 .. run - 1 are drawn, one per tile of
 // the run (a ticket past the run ends the drawing workgroup); whoever reads run - 1 is the
 // last to touch the counter and resets it.
-template <int MODE>
-__global__ __launch_bounds__(big::kThreads) __attribute__((amdgpu_waves_per_eu(2)))
-void gemm_tile_persistent(TileArgs p, int nx) {
-  using namespace big;
-  __shared__ __align__(1024) uint16_t smem[2 * kStage];
-  __shared__ SegTable tab;
-  __shared__ int s_next;
-  load_seg_table<kTM, MODE>(p, tab, nx);
+// walk_tiles is that walk over row tiles of TM rows; tile(loc, hook) computes one tile.
+template <int TM, int MODE, typename Tile>
+__device__ __forceinline__ void walk_tiles(const TileArgs& p, int nx, SegTable& tab, int& s_next,
+                                           Tile tile) {
+  load_seg_table<TM, MODE>(p, tab, nx);
   __syncthreads();
   const int x = blockIdx.x & 7, wpx = gridDim.x >> 3;
   // this XCD's tiles: the x-th eighth of the estimated cost
   const long long ctot = tab.ctotal;
-  const int run0 = tile_at_cost<kTM, MODE>(tab, (int)(ctot * x / 8), nx);
-  const int run = tile_at_cost<kTM, MODE>(tab, (int)(ctot * (x + 1) / 8), nx) - run0;
+  const int run0 = tile_at_cost<TM, MODE>(tab, (int)(ctot * x / 8), nx);
+  const int run = tile_at_cost<TM, MODE>(tab, (int)(ctot * (x + 1) / 8), nx) - run0;
   // a per-lane (to the compiler: divergent) address, so the fetch-add is issued as it stands
   // and its result is waited for only where it is used
   int zero = 0;
@@ -882,7 +880,7 @@ void gemm_tile_persistent(TileArgs p, int nx) {
   while (i < run) {
     const int t = run0 + i;
     const int g = t / nx;
-    const TileLoc loc = seg_tile<kTM>(tab, g, t - g * nx);
+    const TileLoc loc = seg_tile<TM>(tab, g, t - g * nx);
     // (every wave passed the barrier after the previous tile's epilogue, whose LDS reads of the
     // stages had completed: this tile's DMA may refill them)
     auto hook = [&]() {
@@ -895,11 +893,223 @@ void gemm_tile_persistent(TileArgs p, int nx) {
         s_next = nxt;
       }
     };
-    if (loc.rows <= thin::kTM) thin_tile<MODE>(p, loc, smem, hook);
-    else big_tile<MODE>(p, loc, smem, hook);
+    tile(loc, hook);
     __syncthreads();
     i = __builtin_amdgcn_readfirstlane(s_next);
   }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(big::kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_tile_persistent(TileArgs p, int nx) {
+  using namespace big;
+  __shared__ __align__(1024) uint16_t smem[2 * kStage];
+  __shared__ SegTable tab;
+  __shared__ int s_next;
+  walk_tiles<kTM, MODE>(p, nx, tab, s_next, [&](const TileLoc& loc, auto hook) {
+    if (loc.rows <= thin::kTM) thin_tile<MODE>(p, loc, smem, hook);
+    else big_tile<MODE>(p, loc, smem, hook);
+  });
+}
+
+// ================================================================================================
+// Grouped gate/up and down over fp8 e4m3fn expert weights (one fp32 scale per 128 x 128 block) at
+// prefill size: the persistent walk above over 128 x 256 tiles.
+// A K-step is 128 columns, one scale block: 128-byte weight rows (whole cache lines, the same LDS
+// layout as a 64-column bf16 step) and two 64-column sub-tiles of the bf16 activations, all by
+// LDS-DMA. A wave reads 16 weight bytes per lane and converts them to bf16 in registers (exact),
+// so a lane's k order within a 64-column half is 16 kq + 8 m (m = 0, 1 for the low and high 8
+// bytes), which the activation reads follow. The products of a step are summed in a fresh
+// accumulator of one 16-column tile at a time, then scaled in fp32 and added to the output
+// accumulator: the arithmetic of the decode kernels (moe_gemm.hip), no scaled weight is ever
+// rounded.
+// 128 rows per tile and not 256: the activations of a 128-column step are twice a bf16 step's,
+// and two stages of 256 rows do not fit in LDS; and a routed expert has about 100 rows at the
+// sizes this serves. Tiles of at most 64 rows take three stages of 64 rows (two steps of
+// lookahead) with the 8 waves side by side over the columns, so no weight is converted twice.
+// Measured at 3431 tokens, Zipf-skewed over 256 experts of 512 x 2048 (30 879 rows): gate/up
+// 1550 -> 233 us, down 297 -> 168 us against the 16-row passes of the decode kernels.
+// ================================================================================================
+namespace f8 {
+constexpr int kTN = 256, kTK = 128, kThreads = 512;
+constexpr int kTM = 128, kThinTM = 64;
+constexpr int kBElems = kTN * kTK / 2;  // a stage's weight bytes in uint16_t units (32 KB)
+constexpr int stage_elems(int tm) { return tm * kTK + kBElems; }
+constexpr int kSmem = 3 * stage_elems(kThinTM);
+static_assert(kSmem >= 2 * stage_elems(kTM), "both stage rings fit");
+}  // namespace f8
+
+template <int MODE, int TM, typename Hook>
+__device__ __forceinline__ void f8_tile(const TileArgs& p, const TileLoc& loc, uint16_t* smem,
+                                        Hook hook) {
+  using namespace f8;
+  constexpr int WM = TM / 64, WN = 8 / WM;        // waves over rows, columns
+  constexpr int WC = kTN / WN, NJ = WC / 16;      // columns per wave
+  constexpr int kStages = TM == kThinTM ? 3 : 2;
+  constexpr int kAElems = TM * kTK, kStage = stage_elems(TM);
+  constexpr int kAInst = TM / 64;                 // 8-row DMA groups per wave and 64-column half
+  static_assert(MODE != kDense && (MODE == kDown || NJ % 2 == 0), "");
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (opaque, as in thin_tile: per-lane values are not hoisted out of the tile loop)
+  int lane = tid & 63;
+  asm volatile("" : "+v"(lane));
+  const int wm = wave / WN, wn = wave % WN;
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int K = p.K, nk = K / kTK;
+  const int wrows = MODE == kGateUp ? 2 * p.N : p.N;  // weight rows of one expert
+  const uint16_t* wbase =
+      reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(p.w) +
+                                        (size_t)loc.e * wrows * K);
+  // one scale per K-step and 128 weight rows; lane l holds step l's (of 64 at a time). A wave's
+  // columns lie in one 128-row block (GATE_UP: one of gate rows and one of up rows).
+  const float* srow = p.w_scale + (size_t)loc.e * (wrows / 128) * nk;
+  const float* s0 = srow + (size_t)(MODE == kGateUp ? loc.ct : loc.ct * 2 + wn * WC / 128) * nk;
+  const float* s1 = MODE == kGateUp ? s0 + (size_t)(p.N / 128) * nk : s0;
+  float sv0 = s0[min(lane, nk - 1)], sv1 = s1[min(lane, nk - 1)];
+
+  const int lr = lane >> 3;
+  const uint32_t chunk_b = ((lane & 7) ^ lr) * 16;
+  const bool a_on = wave * (TM / 8) < loc.rows;
+  uint32_t b_off[4], a_off[kAInst];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int br = wave * 32 + lr + 8 * i;
+    const int row = MODE == kGateUp ? (br < 128 ? 0 : p.N - 128) + loc.ct * 128 + br
+                                    : loc.ct * kTN + br;
+    b_off[i] = (uint32_t)row * (uint32_t)K + chunk_b;
+  }
+  auto stage_of = [&](int kt) { return smem + (kt % kStages) * kStage; };
+  auto issue_b = [&](int kt) {
+    uint16_t* st = stage_of(kt) + kAElems + wave * 32 * 64;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16(wbase, b_off[i] + (uint32_t)kt * kTK, st + i * 512);
+  };
+  auto issue_a = [&](int kt) {
+    if (!a_on) return;
+    uint16_t* st = stage_of(kt) + wave * (TM / 8) * 64;
+#pragma unroll
+    for (int i = 0; i < kAInst; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        dma16(p.a, a_off[i] + (uint32_t)kt * (2 * kTK) + h * 128, st + h * (TM * 64) + i * 512);
+  };
+  auto rows_of_a = [&]() {
+#pragma unroll
+    for (int i = 0; i < kAInst; ++i)
+      a_off[i] = a_row_offset<MODE>(p, loc, min(wave * (TM / 8) + lr + 8 * i, loc.rows - 1)) +
+                 chunk_b;
+  };
+  // wait for step kt, leaving what was issued after it in flight. Two stages: nothing was.
+  // Three: at kt = 0 (issued B0, B1, A0, A1) step 1's A instructions, or for a wave without A
+  // rows step 1's 4 weight instructions; later step kt + 1's, issued after all of step kt.
+  auto sync_step = [&](int kt) {
+    if (kStages == 2 || kt + 1 >= nk) {
+      SYM_TILE_SYNC(0);
+    } else if (!a_on) {
+      SYM_TILE_SYNC(4);
+    } else if (kt == 0) {
+      SYM_TILE_SYNC(2);
+    } else {
+      SYM_TILE_SYNC(6);
+    }
+  };
+  static_assert(kStages == 2 || kAInst == 1, "sync_step's counts");
+
+  const int ni = min(max((loc.rows - wm * 64 + 15) >> 4, 0), 4);
+  floatx4 acc[4][NJ];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int sw = r16 & 7;
+  const int a_frag = (wm * 64 + r16) * 64;
+  const int b_frag = kAElems + ((MODE == kGateUp ? wn * (WC / 2) : wn * WC) + r16) * 64;
+  auto b_row = [](int j) {
+    return MODE == kGateUp ? (j < NJ / 2 ? 0 : 128) + (j % (NJ / 2)) * 16 : j * 16;
+  };
+  auto loop = [&](auto ni_tag) {
+    constexpr int NI = decltype(ni_tag)::value;
+    issue_b(0);
+    if (kStages > 2 && nk > 1) issue_b(1);
+    rows_of_a();
+    issue_a(0);
+    if (kStages > 2 && nk > 1) issue_a(1);
+    for (int kt = 0; kt < nk; ++kt) {
+      sync_step(kt);
+      // the barrier also means that every wave has read the stage refilled here
+      if (kt + kStages - 1 < nk) {
+        issue_a(kt + kStages - 1);
+        issue_b(kt + kStages - 1);
+      }
+      if (kt > 0 && (kt & 63) == 0) {
+        sv0 = s0[min(kt + lane, nk - 1)];
+        sv1 = s1[min(kt + lane, nk - 1)];
+      }
+      if constexpr (NI > 0) {
+        const uint16_t* st = stage_of(kt);
+        u32x4 a[NI][4];
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk)
+            a[i][kk] = *reinterpret_cast<const u32x4*>(st + a_frag + (kk >> 1) * (TM * 64) +
+                                                       i * 16 * 64 +
+                                                       ((2 * kq + (kk & 1)) ^ sw) * 8);
+        const float c0 = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sv0), kt & 63));
+        const float c1 = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sv1), kt & 63));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          uint4 b[4];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint4 w = *reinterpret_cast<const uint4*>(st + b_frag + b_row(j) * 64 +
+                                                            ((4 * h + kq) ^ sw) * 8);
+            b[2 * h] = fp8x8_to_bf16x8(w.x, w.y);
+            b[2 * h + 1] = fp8x8_to_bf16x8(w.z, w.w);
+          }
+          floatx4 t[NI];
+#pragma unroll
+          for (int i = 0; i < NI; ++i) t[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+              t[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  as_bf16x8(b[kk]), __builtin_bit_cast(bf16x8, a[i][kk]), t[i], 0, 0, 0);
+          const float c = MODE == kGateUp && j >= NJ / 2 ? c1 : c0;
+#pragma unroll
+          for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[i][j][q] = fmaf(c, t[i][q], acc[i][j][q]);
+        }
+      }
+    }
+  };
+  switch (ni) {
+    case 4: loop(std::integral_constant<int, 4>{}); break;
+    case 3: loop(std::integral_constant<int, 3>{}); break;
+    case 2: loop(std::integral_constant<int, 2>{}); break;
+    case 1: loop(std::integral_constant<int, 1>{}); break;
+    default: loop(std::integral_constant<int, 0>{}); break;
+  }
+  hook();
+  const int col0 = MODE == kGateUp ? loc.ct * 128 + wn * (WC / 2) : loc.ct * kTN + wn * WC;
+  if (ni > 0) store_block<MODE, NJ>(p, acc, loc, wm * 64, col0, lane);
+}
+
+template <int MODE>
+__global__ __launch_bounds__(f8::kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_f8_persistent(TileArgs p, int nx) {
+  __shared__ __align__(1024) uint16_t smem[f8::kSmem];
+  __shared__ SegTable tab;
+  __shared__ int s_next;
+  walk_tiles<f8::kTM, MODE>(p, nx, tab, s_next, [&](const TileLoc& loc, auto hook) {
+    if (loc.rows <= f8::kThinTM) f8_tile<MODE, f8::kThinTM>(p, loc, smem, hook);
+    else f8_tile<MODE, f8::kTM>(p, loc, smem, hook);
+  });
 }
 
 // ================================================================================================
@@ -1272,4 +1482,85 @@ extern "C" int sym_moe_down_tiled(const void* h, int T, int H, int I, int rows,
                      dim3((H + C::kTN - 1) / C::kTN, rows / C::kTM + max_segments),
                      dim3(C::kThreads), 0, (hipStream_t)stream, p);
   return sym_host::check_launch("gemm_tile128_kernel");
+}
+
+static int check_grouped_fp8(const char* what, int T, int H, int I, int rows, int max_segments) {
+  int rc = check_grouped(what, T, H, I, rows, max_segments);
+  if (rc) return rc;
+  // tiles of 256 weight rows (128 gate + 128 up) and K-steps of 128 columns, unclamped
+  SYM_REQUIRE(H % 256 == 0 && I % 128 == 0, SYM_ERR_UNSUPPORTED,
+              "%s: H=%d must be a multiple of 256 and I=%d of 128", what, H, I);
+  SYM_REQUIRE(max_segments <= kPersistSeg, SYM_ERR_UNSUPPORTED,
+              "%s: max_segments=%d above %d", what, max_segments, kPersistSeg);
+  return SYM_OK;
+}
+
+extern "C" int sym_moe_gate_up_fp8_tiled(const void* x, int T, int H, int I, int rows,
+                                         const int32_t* sorted_tokens, const int32_t* seg_expert,
+                                         const int32_t* seg_offset, const int32_t* seg_count,
+                                         const int32_t* n_segments, int max_segments,
+                                         const void* w_gate_up, const float* s_gate_up, void* h,
+                                         void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_grouped_fp8("moe_gate_up_fp8_tiled", T, H, I, rows, max_segments);
+  if (!rc) rc = check_tickets("moe_gate_up_fp8_tiled", workspace, workspace_bytes);
+  if (rc || rows == 0 || T == 0) return rc;
+  SYM_REQUIRE(x && sorted_tokens && seg_expert && seg_offset && seg_count && n_segments &&
+                  w_gate_up && s_gate_up && h,
+              SYM_ERR_INVALID, "moe_gate_up_fp8_tiled: null pointer argument");
+  SYM_REQUIRE(aligned(x, 16) && aligned(w_gate_up, 16) && aligned(s_gate_up, 4) && aligned(h, 16),
+              SYM_ERR_INVALID, "moe_gate_up_fp8_tiled: x, w_gate_up and h must be 16-byte aligned");
+  TileArgs p{};
+  p.a = (const uint16_t*)x;
+  p.w = (const uint16_t*)w_gate_up;
+  p.w_scale = s_gate_up;
+  p.sorted_tokens = sorted_tokens;
+  p.seg_expert = seg_expert;
+  p.seg_offset = seg_offset;
+  p.seg_count = seg_count;
+  p.n_segments = n_segments;
+  p.max_segments = max_segments;
+  p.M = rows;
+  p.N = I;
+  p.K = H;
+  p.out_bf16 = (uint16_t*)h;
+  p.tickets = (int*)workspace;
+  (void)hipGetLastError();
+  const int grid = std::max(8, sym_host::cu_count() / 8 * 8);
+  hipLaunchKernelGGL((gemm_f8_persistent<kGateUp>), dim3(grid), dim3(f8::kThreads), 0,
+                     (hipStream_t)stream, p, I / 128);
+  return sym_host::check_launch("gemm_f8_persistent");
+}
+
+extern "C" int sym_moe_down_fp8_tiled(const void* h, int T, int H, int I, int rows,
+                                      const int32_t* seg_expert, const int32_t* seg_offset,
+                                      const int32_t* seg_count, const int32_t* n_segments,
+                                      int max_segments, const void* w_down, const float* s_down,
+                                      float* y, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+  int rc = check_grouped_fp8("moe_down_fp8_tiled", T, H, I, rows, max_segments);
+  if (!rc) rc = check_tickets("moe_down_fp8_tiled", workspace, workspace_bytes);
+  if (rc || rows == 0 || T == 0) return rc;
+  SYM_REQUIRE(h && seg_expert && seg_offset && seg_count && n_segments && w_down && s_down && y,
+              SYM_ERR_INVALID, "moe_down_fp8_tiled: null pointer argument");
+  SYM_REQUIRE(aligned(h, 16) && aligned(w_down, 16) && aligned(s_down, 4) && aligned(y, 16),
+              SYM_ERR_INVALID, "moe_down_fp8_tiled: h, w_down and y must be 16-byte aligned");
+  TileArgs p{};
+  p.a = (const uint16_t*)h;
+  p.w = (const uint16_t*)w_down;
+  p.w_scale = s_down;
+  p.seg_expert = seg_expert;
+  p.seg_offset = seg_offset;
+  p.seg_count = seg_count;
+  p.n_segments = n_segments;
+  p.max_segments = max_segments;
+  p.M = rows;
+  p.N = H;
+  p.K = I;
+  p.out_f32 = y;
+  p.tickets = (int*)workspace;
+  (void)hipGetLastError();
+  const int grid = std::max(8, sym_host::cu_count() / 8 * 8);
+  hipLaunchKernelGGL((gemm_f8_persistent<kDown>), dim3(grid), dim3(f8::kThreads), 0,
+                     (hipStream_t)stream, p, H / f8::kTN);
+  return sym_host::check_launch("gemm_f8_persistent");
 }
