@@ -453,6 +453,37 @@ def test_gemm_tiled(device, M, N, K, bias, res, out_dtype):
         _close(out, ref, atol=2e-3, rtol=8e-3)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 16, 64), (31, 3072, 2048), (33, 2048, 128),       # 32 x 64 tiles, one or two K-steps
+    (65, 4096, 192), (300, 3072, 256), (512, 3056, 320),  # 64 x 64
+    (1000, 2064, 256), (900, 2048, 448),                  # 64 x 128
+    (1500, 3072, 64), (2101, 2048, 5120), (5400, 3088, 128),  # 128 x 128
+    (17, 131200, 1024), (50, 131216, 1024), (129, 131088, 1088),  # weights over 256 MB
+])
+@pytest.mark.parametrize("kind", ["bf16", "f32", "bias_res32", "res16"])
+def test_gemm_small_tiles(device, M, N, K, kind):
+    """Row and column remainders of the small dense tiles, with every epilogue, against fp32."""
+    if N > 100000 and kind != "f32":
+        pytest.skip("one output type of the large weights is enough")
+    g = torch.Generator(device=device).manual_seed(M + N)
+    a = torch.randn(M, K, generator=g, device=device).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=device) * 0.05).bfloat16()
+    want = a.float() @ w.float().T
+    kw = {"out_dtype": torch.bfloat16 if kind in ("bf16", "bias_res32") else torch.float32}
+    if kind == "bias_res32":
+        kw["bias"] = torch.randn(N, generator=g, device=device).bfloat16()
+        kw["residual"] = torch.randn(M, N, generator=g, device=device)
+        want = want + kw["bias"].float() + kw["residual"]
+    if kind == "res16":
+        kw["residual"] = torch.randn(M, N, generator=g, device=device).bfloat16()
+        want = want + kw["residual"].float()
+    out = torch.full((M, N), float("nan"), dtype=kw["out_dtype"], device=device)
+    hip_ops.gemm(a, w, out=out, **kw)
+    # fp32 sums of K products of magnitude ~0.05 in another order, then one bf16 rounding (2^-9)
+    rtol = 2 ** -8 if kw["out_dtype"] == torch.bfloat16 else 1e-5
+    torch.testing.assert_close(out.float(), want, rtol=rtol, atol=1e-4)
+
+
 @pytest.mark.parametrize("M,N,K,bias", [(9942, 2048, 2048, False), (77, 400, 192, True),
                                         (8500, 2048, 128, True)])
 def test_gemm_tiled_bf16_residual(device, M, N, K, bias):

@@ -18,6 +18,7 @@
 //     overlap the other half's MFMAs, with one barrier per step. In the persistent kernels a
 //     tile of at most 64 valid rows runs thin_tile instead: three 40 KB stages (64 A rows and
 //     256 B rows each), two steps of lookahead.
+//   gemm_small_kernel: 32 x 64 to 128 x 256 tiles for dense GEMMs of few rows (dense_tiling).
 //   gemm_tile128_kernel (router logits, N = E = 256: few tiles; grouped down projection over
 //     longer segment lists): 128 x 256 tiles, two workgroups of 8 waves per CU, each
 //     wave a 64 x 64 block; 32 columns per step through a 3-stage 72 KB ring. The second
@@ -73,6 +74,7 @@ struct TileArgs {
   long long out_zstride;    // ... and output plane out + z * out_zstride (elements)
   int full_rt;              // DENSE with tail_rows > 0: row tiles 0 .. full_rt - 1 have TM rows,
   int tail_rows;            // the rows from full_rt * TM on tiles of tail_rows (one plane)
+  int col_major;            // DENSE: the row tiles of a column tile are neighbours (N > M)
   int* tickets;             // persistent grids: the caller's 8 per-XCD tile counters
   const float* w_scale;     // fp8 weights: [S, rows / 128, K / 128] block scales
 };
@@ -88,6 +90,10 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // in flight.
 #define SYM_TILE_SYNC(N) \
   asm volatile("s_waitcnt vmcnt(" #N ")\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
+
+// The same with a constant expression for the count.
+#define SYM_TILE_SYNC_N(N) \
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory")
 
 // Tile t of n for the workgroup with linear id lin, or -1. Workgroups are dispatched to the 8
 // XCDs round-robin by linear id (lin % 8), and each XCD has its own L2: XCD x takes the
@@ -132,8 +138,9 @@ __device__ __forceinline__ bool locate_tile(const TileArgs& p, int lane, TileLoc
     }
     const int t = xcd_tile(lin, nxy * gridDim.z);  // the grid holds exactly the tiles
     loc.z = t / nxy;
-    const int gy = (t - loc.z * nxy) / nx;
-    loc.ct = t - loc.z * nxy - gy * nx;
+    const int tz = t - loc.z * nxy;
+    const int gy = p.col_major ? tz % (int)gridDim.y : tz / nx;
+    loc.ct = p.col_major ? tz / (int)gridDim.y : tz - gy * nx;
     loc.row0 = gy * TM;
     loc.rows = min(TM, p.M - loc.row0);
     return true;
@@ -242,8 +249,8 @@ __device__ __forceinline__ uint32_t a_row_offset(const TileArgs& p, const TileLo
 // columns; h = silu(gate) * up. Otherwise tile j is columns col0 + 16 j ..
 // The 4 output values of tile (i, j) held by this lane, for output row orow and first column
 // col (col < N): GATE_UP h, DENSE plus bias and residual, DOWN as computed.
-template <int MODE, int NJ>
-__device__ __forceinline__ void tile_values(const TileArgs& p, const floatx4 (&acc)[4][NJ], int i,
+template <int MODE, int NJ, int NI>
+__device__ __forceinline__ void tile_values(const TileArgs& p, const floatx4 (&acc)[NI][NJ], int i,
                                             int j, size_t orow, int col, float (&v)[4]) {
   if constexpr (MODE == kGateUp) {
 #pragma unroll
@@ -272,13 +279,13 @@ __device__ __forceinline__ void tile_values(const TileArgs& p, const floatx4 (&a
 
 // Direct epilogue: each (i, j) tile as one 8-byte (bf16) or 16-byte (fp32) write per lane, i.e.
 // an instruction writes 32 or 64 bytes into each of 16 rows.
-template <int MODE, int NJ>
-__device__ __forceinline__ void store_block(const TileArgs& p, const floatx4 (&acc)[4][NJ],
+template <int MODE, int NJ, int NI>
+__device__ __forceinline__ void store_block(const TileArgs& p, const floatx4 (&acc)[NI][NJ],
                                             const TileLoc& loc, int rbase, int col0, int lane) {
   const int r16 = lane & 15, kq = lane >> 4;
   constexpr int NT = MODE == kGateUp ? NJ / 2 : NJ;  // output tiles per 16-row sub-tile
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NI; ++i) {
     const int r = rbase + i * 16 + r16;
     if (r >= loc.rows) continue;
     const size_t orow = (size_t)(loc.row0 + r);
@@ -299,7 +306,7 @@ __device__ __forceinline__ void store_block(const TileArgs& p, const floatx4 (&a
       const int col = col0 + j * 16 + kq * 4;
       if (col >= p.N) continue;  // N % 16 == 0: the 4 columns are all valid or all not
       float v[4];
-      tile_values<MODE, NJ>(p, acc, i, j, orow, col, v);
+      tile_values<MODE>(p, acc, i, j, orow, col, v);
       if constexpr (MODE == kDense) {
         if (p.residual_bf16) {
           v[0] += bf16_lo(rb[j].x); v[1] += bf16_hi(rb[j].x);
@@ -354,7 +361,7 @@ __device__ __forceinline__ void store_block_lds(const TileArgs& p, const floatx4
       const int col = col0 + j * 16 + kq * 4;
       if (row >= nrows || col >= p.N) continue;
       float v[4];
-      tile_values<MODE, NJ>(p, acc, i, j, orow, col, v);
+      tile_values<MODE>(p, acc, i, j, orow, col, v);
       *reinterpret_cast<uint2*>(buf + slot(row, 2 * j + (kq >> 1)) + (kq & 1) * 4) =
           make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     }
@@ -561,7 +568,7 @@ __device__ __forceinline__ void big_tile(TileArgs p, const TileLoc& loc, uint16_
     constexpr int kBlockElems = 64 * (MODE == kGateUp ? kWC / 2 : kWC);
     store_block_lds<MODE, kNJ>(p, acc, loc, wm * 64, col0, lane, smem + wave * kBlockElems);
   } else if (m_on) {
-    store_block<MODE, kNJ>(p, acc, loc, wm * 64, col0, lane);
+    store_block<MODE>(p, acc, loc, wm * 64, col0, lane);
   }
 }
 
@@ -709,7 +716,7 @@ __device__ __forceinline__ void thin_tile(TileArgs p, const TileLoc& loc, uint16
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     store_block_lds<MODE, kNJ>(p, acc, loc, m_on ? 0 : 64, col0, lane, smem + wave * 64 * kCols);
   } else if (m_on) {
-    store_block<MODE, kNJ>(p, acc, loc, 0, col0, lane);
+    store_block<MODE>(p, acc, loc, 0, col0, lane);
   }
 }
 
@@ -1097,7 +1104,7 @@ __device__ __forceinline__ void f8_tile(const TileArgs& p, const TileLoc& loc, u
   }
   hook();
   const int col0 = MODE == kGateUp ? loc.ct * 128 + wn * (WC / 2) : loc.ct * kTN + wn * WC;
-  if (ni > 0) store_block<MODE, NJ>(p, acc, loc, wm * 64, col0, lane);
+  if (ni > 0) store_block<MODE>(p, acc, loc, wm * 64, col0, lane);
 }
 
 template <int MODE>
@@ -1229,7 +1236,108 @@ void gemm_tile128_kernel(TileArgs p) {
   if (ni == 0) return;
 
   const int col0 = MODE == kGateUp ? loc.ct * (kTN / 2) + wn * (kWC / 2) : loc.ct * kTN + wn * kWC;
-  store_block<MODE, kNJ>(p, acc, loc, wm * 64, col0, lane);
+  store_block<MODE>(p, acc, loc, wm * 64, col0, lane);
+}
+
+// ================================================================================================
+// Small tiles (32 x 64 up to 128 x 256) for dense GEMMs whose 256 x 256 tiles leave most of the
+// chip idle: a WM x WN grid of waves per workgroup, 64-column steps through an S-stage LDS ring
+// (S - 1 steps of lookahead, one barrier per step), up to 3 independent workgroups per CU that
+// cover each other's waits. With few tiles a K-step costs a memory round trip divided by the
+// lookahead, so the smallest tiles that fill the chip are the fastest; with many, the operands'
+// L2 traffic bounds the small tiles (dense_tiling has the measurements).
+// ================================================================================================
+namespace small {
+constexpr int kTK = 64;
+constexpr int stage_elems(int tm, int tn) { return (tm + tn) * kTK; }
+}  // namespace small
+
+template <int MODE, int TM, int TN, int S, int WM = 2, int WN = 2>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_small_kernel(TileArgs p) {
+  using namespace small;
+  constexpr int kW = WM * WN, kWR = TM / WM, kWC = TN / WN;  // waves; rows, columns of each
+  constexpr int NI = kWR / 16, NJ = kWC / 16;
+  constexpr int kStage = stage_elems(TM, TN), kAElems = TM * kTK;
+  constexpr int kADma = TM / (8 * kW), kBDma = TN / (8 * kW), kDma = kADma + kBDma;  // per wave and step
+  __shared__ __align__(1024) uint16_t smem[S * kStage];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave / WN, wn = wave % WN;
+  const int r16 = lane & 15, kq = lane >> 4;
+  TileLoc loc;
+  if (!locate_tile<kDense, TM>(p, lane, loc)) return;
+  const uint16_t* wbase = tile_weights<kDense>(p, loc);
+
+  const int lr = lane >> 3;
+  const uint32_t chunk_b = ((lane & 7) ^ lr) * 16;
+  uint32_t a_off[kADma], b_off[kBDma];
+#pragma unroll
+  for (int i = 0; i < kBDma; ++i)
+    b_off[i] = b_row_offset<MODE, TN>(p, loc.ct, wave * (TN / kW) + lr + 8 * i) + chunk_b;
+#pragma unroll
+  for (int i = 0; i < kADma; ++i)
+    a_off[i] = a_row_offset<kDense>(p, loc, min(wave * (TM / kW) + lr + 8 * i, loc.rows - 1)) +
+               chunk_b;
+  auto issue = [&](int kt) {
+    uint16_t* st = smem + (kt % S) * kStage;
+    const uint32_t k = (uint32_t)kt * (kTK * 2);
+#pragma unroll
+    for (int i = 0; i < kBDma; ++i)
+      dma16(wbase, b_off[i] + k, st + kAElems + (wave * (TN / kW) + 8 * i) * kTK);
+#pragma unroll
+    for (int i = 0; i < kADma; ++i) dma16(p.a, a_off[i] + k, st + (wave * (TM / kW) + 8 * i) * kTK);
+  };
+  const int sw = r16 & 7;
+  const int a_frag = (wm * kWR + r16) * kTK;
+  const int b_frag = kAElems + ((MODE == kGateUp ? wn * (kWC / 2) : wn * kWC) + r16) * kTK;
+  auto b_row = [](int j) {
+    return MODE == kGateUp ? (j < NJ / 2 ? 0 : TN / 2) + (j % (NJ / 2)) * 16 : j * 16;
+  };
+  floatx4 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  const int nk = p.K / kTK;
+#pragma unroll
+  for (int i = 0; i < S - 1; ++i)
+    if (i < nk) issue(i);
+  for (int kt = 0; kt < nk; ++kt) {
+    // wait for step kt; the steps issued after it stay in flight
+    const int rem = min(nk - 1 - kt, S - 2);
+    if (rem <= 0) SYM_TILE_SYNC_N(0);
+    else if (rem == 1) SYM_TILE_SYNC_N(kDma);
+    else if (rem == 2) SYM_TILE_SYNC_N(2 * kDma);
+    else if (rem == 3) SYM_TILE_SYNC_N(3 * kDma);
+    else SYM_TILE_SYNC_N(4 * kDma);
+    // the barrier also means that every wave has read the stage refilled here
+    if (kt + S - 1 < nk) issue(kt + S - 1);
+    const uint16_t* st = smem + (kt % S) * kStage;
+    u32x4 a[2][NI], b[2][NJ];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int slot = ((4 * h + kq) ^ sw) * 8;
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        a[h][i] = *reinterpret_cast<const u32x4*>(st + a_frag + i * 16 * kTK + slot);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        b[h][j] = *reinterpret_cast<const u32x4*>(st + b_frag + b_row(j) * kTK + slot);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, b[h][j]), __builtin_bit_cast(bf16x8, a[h][i]),
+              acc[i][j], 0, 0, 0);
+  }
+  const int col0 = MODE == kGateUp ? loc.ct * (TN / 2) + wn * (kWC / 2) : loc.ct * TN + wn * kWC;
+  store_block<MODE>(p, acc, loc, wm * kWR, col0, lane);
 }
 
 }  // namespace sym
@@ -1279,6 +1387,49 @@ static void dense_tail_split(int M, int nx, int cus, int& full_rt, int& tail_row
   }
 }
 
+// Which tiles a dense GEMM runs on.
+// A weight too large for the caches (over 256 MB, e.g. an LM head) streams from HBM whatever the
+// tile, so the one with the fewest operand re-reads that covers M is taken (157184 x 2048, us,
+// 256 x 256 tiles against the choice): 32 rows 161 / 126 on 32 x 64; 64: 176 / 135 on 64 x 128;
+// 96: 189 / 160, 128: 198 / 168, 256: 272 / 214 on 128 x 256 (16: 154 / 119).
+// Otherwise by estimated time: at K = 2048 a workgroup alone on its CU takes `alone` us and each
+// further one on the busiest CU `more`, with the load halfway between the mean and the busiest
+// CU's (fitted to sweeps of M = 16 .. 9322 at N = 2048 and 3072, K = 2048 and 5120; time scales
+// with K). Measured (us, 256 x 256 against the choice) for N x K = 3072 x 2048: M = 64 27.6 /
+// 10.0, 333 32.2 / 13.9, 512 31.8 / 14.7, 1024 33.4 / 22.1, 1710 33.8 / 32.3; 256 x 256 stays for
+// 2560-5000 (46.2 / 54.9 at 3431) and from 5600 rows (101.5 / 120.5 at 9322).
+enum DenseTiles { kTiles32x64, kTiles64x64, kTiles64x128, kTiles128x128, kTiles128x256, kTiles256 };
+static DenseTiles dense_tiling(int M, int N, int K, int cus) {
+  if ((long long)N * K * 2 > (256ll << 20) && M <= 256)
+    return M <= 32 ? kTiles32x64 : M <= 64 ? kTiles64x128 : kTiles128x256;
+  struct Kind {
+    DenseTiles id;
+    int tm, tn;
+    double alone, more;
+  };
+  static const Kind kinds[] = {{kTiles32x64, 32, 64, 10.0, 4.4},
+                               {kTiles64x64, 64, 64, 11.0, 6.5},
+                               {kTiles64x128, 64, 128, 15.0, 9.0},
+                               {kTiles128x128, 128, 128, 20.0, 16.5}};
+  const long long big_tiles = (long long)((M + 255) / 256) * ((N + 255) / 256);
+  double best = big_tiles <= cus ? 30.0 + 16.0 * big_tiles / cus
+                                 // 50 a round, less what dense_tail_split may save
+                                 : 40.0 * ((big_tiles + cus - 1) / cus);
+  DenseTiles id = kTiles256;
+  for (const Kind& k : kinds) {
+    const long long rt = (M + k.tm - 1) / k.tm, tiles = rt * ((N + k.tn - 1) / k.tn);
+    if (rt > 65535) continue;
+    const double mean = std::max(1.0, (double)tiles / cus);
+    const double load = 0.5 * (mean + (double)((tiles + cus - 1) / cus));
+    const double est = k.alone + k.more * (load - 1.0);
+    if (est < best) {
+      best = est;
+      id = k.id;
+    }
+  }
+  return id;
+}
+
 static int gemm_dense(const char* what, const void* a, const void* w, const void* bias,
                       const float* residual, const void* residual_bf16, int M, int N, int K,
                       void* out, int out_fp32, void* stream) {
@@ -1309,13 +1460,28 @@ static int gemm_dense(const char* what, const void* a, const void* w, const void
   p.K = K;
   p.out_bf16 = out_fp32 ? nullptr : (uint16_t*)out;
   p.out_f32 = out_fp32 ? (float*)out : nullptr;
+  (void)hipGetLastError();
+  const int cus = sym_host::cu_count();
+  hipStream_t s = (hipStream_t)stream;
+#define SYM_LAUNCH_SMALL(TM, TN, S, WM, WN)                                                      \
+  p.col_major = N > M;                                                                           \
+  hipLaunchKernelGGL((gemm_small_kernel<kDense, TM, TN, S, WM, WN>),                             \
+                     dim3((N + TN - 1) / TN, (M + TM - 1) / TM), dim3(64 * WM * WN), 0, s, p);   \
+  return sym_host::check_launch("gemm_small_kernel")
+  switch (dense_tiling(M, N, K, cus)) {
+    case kTiles32x64: SYM_LAUNCH_SMALL(32, 64, 4, 2, 2);
+    case kTiles64x64: SYM_LAUNCH_SMALL(64, 64, 3, 2, 2);
+    case kTiles64x128: SYM_LAUNCH_SMALL(64, 128, 3, 2, 4);
+    case kTiles128x128: SYM_LAUNCH_SMALL(128, 128, 2, 2, 4);
+    case kTiles128x256: SYM_LAUNCH_SMALL(128, 256, 3, 2, 4);
+    default: break;
+  }
+#undef SYM_LAUNCH_SMALL
   const int nx = (N + C::kTN - 1) / C::kTN;
   int rt = (M + C::kTM - 1) / C::kTM;
-  dense_tail_split(M, nx, sym_host::cu_count(), p.full_rt, p.tail_rows);
+  dense_tail_split(M, nx, cus, p.full_rt, p.tail_rows);
   if (p.tail_rows > 0) rt = p.full_rt + (M - p.full_rt * C::kTM + p.tail_rows - 1) / p.tail_rows;
-  (void)hipGetLastError();
-  hipLaunchKernelGGL((gemm_tile_kernel<kDense>), dim3(nx, rt), dim3(C::kThreads), 0,
-                     (hipStream_t)stream, p);
+  hipLaunchKernelGGL((gemm_tile_kernel<kDense>), dim3(nx, rt), dim3(C::kThreads), 0, s, p);
   return sym_host::check_launch("gemm_tile_kernel");
 }
 
