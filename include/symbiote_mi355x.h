@@ -372,8 +372,8 @@ int sym_moe_down_fp8(const void* h, int T, int H, int I, const int32_t* seg_expe
                      const float* s_down, float* y, void* stream);
 
 /* ---------------------------------------------------------------------------------------
- * Tiled GEMMs for prefill-size batches (MFMA-bound; 256 x 256 output tiles, 128 x 256 for the
- * grouped down projection over segment lists of more than 512 entries).
+ * Tiled GEMMs for prefill-size batches (MFMA-bound; 256 x 256 output tiles, 32 x 64 to 128 x 256
+ * for dense products of few rows, 128 x 256 for the grouped down projection over segment lists of more than 512 entries).
  * sym_gemm_bf16: out[M, N] = a[M, K] . w[N, K]^T (+ bias[N] bf16) (+ residual[M, N] fp32),
  *   bf16 out, or fp32 when out_fp32 != 0. Replaces the QKV / dense projections at sequence length
  *   > 1 (ttnn_attention.py:2001-2011, 2153-2230). N % 16 == 0, K % 64 == 0; a, w, out and
@@ -382,6 +382,9 @@ int sym_moe_down_fp8(const void* h, int T, int H, int I, const int32_t* seg_expe
  *   taken in fp32 in the epilogue: the dense projection plus the decoder layer's first residual
  *   add at sequence length > 1 (ttnn_attention.py:2211-2230 dense, modeling_bailing_moe_v2.py:
  *   457-460 residual). Same shape rules as sym_gemm_bf16; residual 8-byte aligned.
+ * sym_gemm_swiglu_bf16: h[M, I] = silu(x . w[:I]^T) * (x . w[I:]^T) (bf16, w [2I, K]): the gate and
+ *   up projections of a dense MLP (TTNNBailingMoeV2MLP) in one product. I % 64 == 0, K % 64 == 0;
+ *   x, w and h 16-byte aligned; x and w each under 4 GB.
  * sym_moe_gate_up_tiled / sym_moe_down_tiled: the grouped expert GEMMs of sym_moe_gate_up /
  *   sym_moe_down (same arguments and results; TTNNExperts.forward, ttnn_moe.py:1250-1289) for
  *   segments of many rows; rows = total rows of the segment list (T*top_k + T with the shared
@@ -404,6 +407,7 @@ int sym_gemm_bf16(const void* a, const void* w, const void* bias, const float* r
                   int N, int K, void* out, int out_fp32, void* stream);
 int sym_gemm_bf16_res_bf16(const void* a, const void* w, const void* bias, const void* residual,
                            int M, int N, int K, float* out, void* stream);
+int sym_gemm_swiglu_bf16(const void* x, const void* w, int M, int I, int K, void* h, void* stream);
 int sym_moe_gate_up_tiled(const void* x, int T, int H, int I, int rows,
                           const int32_t* sorted_tokens, const int32_t* seg_expert,
                           const int32_t* seg_offset, const int32_t* seg_count,

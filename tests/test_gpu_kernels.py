@@ -14,6 +14,7 @@ import torch.nn.functional as F
 
 from oracle import route as R
 from oracle.paged_kv import paged_decode_ref
+import tt_symbiote_amd as ts
 from tt_symbiote_amd import hip_ops
 from tt_symbiote_amd.modules.kv_cache import HIPPagedAttentionKVCache, PagedAttentionConfig
 from tt_symbiote_amd.workloads import paged_context
@@ -482,6 +483,31 @@ def test_gemm_small_tiles(device, M, N, K, kind):
     # fp32 sums of K products of magnitude ~0.05 in another order, then one bf16 rounding (2^-9)
     rtol = 2 ** -8 if kw["out_dtype"] == torch.bfloat16 else 1e-5
     torch.testing.assert_close(out.float(), want, rtol=rtol, atol=1e-4)
+
+
+@pytest.mark.parametrize("M,I,H", [
+    (1, 64, 256), (31, 192, 512), (64, 5120, 2048),       # 32 x 64 / 64 x 64 tiles
+    (129, 5120, 256), (300, 5120, 256), (700, 4992, 256),  # 64 x 128, 128 x 128
+    (3001, 5120, 256),                                    # 256 x 256
+])
+def test_dense_mlp(device, M, I, H):
+    """HIPBailingMoeV2MLP over the tile kinds of its products, against fp32 with h rounded to
+    bf16 as the module does; with and without the residual."""
+    g = torch.Generator(device=device).manual_seed(M + I)
+    x = torch.randn(M, H, generator=g, device=device).bfloat16()
+    gate, up = ((torch.randn(I, H, generator=g, device=device) * 0.05).bfloat16()
+                for _ in range(2))
+    down = (torch.randn(H, I, generator=g, device=device) * 0.05).bfloat16()
+    res = torch.randn(M, H, generator=g, device=device)
+    mlp = ts.HIPBailingMoeV2MLP.from_weights(gate, up, down)
+    ts.set_device(mlp, device)
+    h = hip_ops.gemm_swiglu(x, torch.cat([gate, up]))
+    h_ref = F.silu(x.float() @ gate.float().T) * (x.float() @ up.float().T)
+    # one bf16 rounding (2^-9) of an fp32 value
+    torch.testing.assert_close(h.float(), h_ref, rtol=2 ** -8, atol=1e-4)
+    want = h.float() @ down.float().T
+    torch.testing.assert_close(mlp(x).float(), want, rtol=2 ** -8, atol=1e-3)
+    torch.testing.assert_close(mlp(x, residual=res).float(), want + res, rtol=2 ** -8, atol=1e-3)
 
 
 @pytest.mark.parametrize("M,N,K,bias", [(9942, 2048, 2048, False), (77, 400, 192, True),

@@ -233,12 +233,14 @@ __device__ __forceinline__ uint32_t b_row_offset(const TileArgs& p, int ct, int 
   return brow * (uint32_t)p.K * 2u;
 }
 
-// Byte offset of A row r (< rows) of the tile: GATE_UP gathers x[sorted_tokens[row]].
+// Byte offset of A row r (< rows) of the tile: GATE_UP gathers x[sorted_tokens[row]] (a dense
+// MLP has no sorted_tokens: its rows are x's).
 template <int MODE>
 __device__ __forceinline__ uint32_t a_row_offset(const TileArgs& p, const TileLoc& loc, int r) {
-  uint32_t arow;
-  if constexpr (MODE == kGateUp) arow = (uint32_t)p.sorted_tokens[loc.row0 + r];
-  else arow = (uint32_t)(loc.row0 + r);
+  uint32_t arow = (uint32_t)(loc.row0 + r);
+  if constexpr (MODE == kGateUp) {
+    if (p.sorted_tokens) arow = (uint32_t)p.sorted_tokens[arow];
+  }
   return arow * (uint32_t)p.K * 2u;
 }
 
@@ -728,6 +730,16 @@ void gemm_tile_kernel(TileArgs p) {
   TileLoc loc;
   if (!locate_tile<MODE, kTM>(p, threadIdx.x & 63, loc)) return;
   big_tile<MODE>(p, loc, smem);
+}
+
+// gate/up + SwiGLU of a dense MLP (one weight, rows of x in order) on the 256 x 256 tiles.
+__global__ __launch_bounds__(big::kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_swiglu_kernel(TileArgs p) {
+  using namespace big;
+  __shared__ __align__(1024) uint16_t smem[2 * kStage];
+  TileLoc loc;
+  if (!locate_tile<kDense, kTM>(p, threadIdx.x & 63, loc)) return;
+  big_tile<kGateUp>(p, loc, smem);
 }
 
 // Segment list of the grouped modes in LDS (at most kPersistSeg segments): the first row tile
@@ -1399,8 +1411,8 @@ static void dense_tail_split(int M, int nx, int cus, int& full_rt, int& tail_row
 // 10.0, 333 32.2 / 13.9, 512 31.8 / 14.7, 1024 33.4 / 22.1, 1710 33.8 / 32.3; 256 x 256 stays for
 // 2560-5000 (46.2 / 54.9 at 3431) and from 5600 rows (101.5 / 120.5 at 9322).
 enum DenseTiles { kTiles32x64, kTiles64x64, kTiles64x128, kTiles128x128, kTiles128x256, kTiles256 };
-static DenseTiles dense_tiling(int M, int N, int K, int cus) {
-  if ((long long)N * K * 2 > (256ll << 20) && M <= 256)
+static DenseTiles dense_tiling(int M, int N, int K, int cus, bool dense) {
+  if (dense && (long long)N * K * 2 > (256ll << 20) && M <= 256)
     return M <= 32 ? kTiles32x64 : M <= 64 ? kTiles64x128 : kTiles128x256;
   struct Kind {
     DenseTiles id;
@@ -1414,7 +1426,7 @@ static DenseTiles dense_tiling(int M, int N, int K, int cus) {
   const long long big_tiles = (long long)((M + 255) / 256) * ((N + 255) / 256);
   double best = big_tiles <= cus ? 30.0 + 16.0 * big_tiles / cus
                                  // 50 a round, less what dense_tail_split may save
-                                 : 40.0 * ((big_tiles + cus - 1) / cus);
+                                 : (dense ? 40.0 : 50.0) * ((big_tiles + cus - 1) / cus);
   DenseTiles id = kTiles256;
   for (const Kind& k : kinds) {
     const long long rt = (M + k.tm - 1) / k.tm, tiles = rt * ((N + k.tn - 1) / k.tn);
@@ -1428,6 +1440,25 @@ static DenseTiles dense_tiling(int M, int N, int K, int cus) {
     }
   }
   return id;
+}
+
+// Small tiles of a dense product with nw weight rows (GATE_UP: 2 N).
+template <int MODE>
+static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s) {
+  p.col_major = nw > p.M;
+#define SYM_LAUNCH_SMALL(TM, TN, S, WM, WN)                                                      \
+  hipLaunchKernelGGL((gemm_small_kernel<MODE, TM, TN, S, WM, WN>),                               \
+                     dim3((nw + TN - 1) / TN, (p.M + TM - 1) / TM), dim3(64 * WM * WN), 0, s, p); \
+  break
+  switch (id) {
+    case kTiles32x64: SYM_LAUNCH_SMALL(32, 64, 4, 2, 2);
+    case kTiles64x64: SYM_LAUNCH_SMALL(64, 64, 3, 2, 2);
+    case kTiles64x128: SYM_LAUNCH_SMALL(64, 128, 3, 2, 4);
+    case kTiles128x128: SYM_LAUNCH_SMALL(128, 128, 2, 2, 4);
+    default: SYM_LAUNCH_SMALL(128, 256, 3, 2, 4);
+  }
+#undef SYM_LAUNCH_SMALL
+  return sym_host::check_launch("gemm_small_kernel");
 }
 
 static int gemm_dense(const char* what, const void* a, const void* w, const void* bias,
@@ -1463,20 +1494,8 @@ static int gemm_dense(const char* what, const void* a, const void* w, const void
   (void)hipGetLastError();
   const int cus = sym_host::cu_count();
   hipStream_t s = (hipStream_t)stream;
-#define SYM_LAUNCH_SMALL(TM, TN, S, WM, WN)                                                      \
-  p.col_major = N > M;                                                                           \
-  hipLaunchKernelGGL((gemm_small_kernel<kDense, TM, TN, S, WM, WN>),                             \
-                     dim3((N + TN - 1) / TN, (M + TM - 1) / TM), dim3(64 * WM * WN), 0, s, p);   \
-  return sym_host::check_launch("gemm_small_kernel")
-  switch (dense_tiling(M, N, K, cus)) {
-    case kTiles32x64: SYM_LAUNCH_SMALL(32, 64, 4, 2, 2);
-    case kTiles64x64: SYM_LAUNCH_SMALL(64, 64, 3, 2, 2);
-    case kTiles64x128: SYM_LAUNCH_SMALL(64, 128, 3, 2, 4);
-    case kTiles128x128: SYM_LAUNCH_SMALL(128, 128, 2, 2, 4);
-    case kTiles128x256: SYM_LAUNCH_SMALL(128, 256, 3, 2, 4);
-    default: break;
-  }
-#undef SYM_LAUNCH_SMALL
+  if (const DenseTiles id = dense_tiling(M, N, K, cus, true); id != kTiles256)
+    return launch_small<kDense>(id, p, N, s);
   const int nx = (N + C::kTN - 1) / C::kTN;
   int rt = (M + C::kTM - 1) / C::kTM;
   dense_tail_split(M, nx, cus, p.full_rt, p.tail_rows);
@@ -1496,6 +1515,44 @@ extern "C" int sym_gemm_bf16_res_bf16(const void* a, const void* w, const void* 
   SYM_REQUIRE(M <= 0 || residual, SYM_ERR_INVALID, "gemm_bf16_res_bf16: null residual");
   return gemm_dense("gemm_bf16_res_bf16", a, w, bias, nullptr, residual, M, N, K, out, 1,
                     stream);
+}
+
+// h[M, I] = silu(x Wg^T) * (x Wu^T) of a dense MLP, w [2I, K] with the gate rows first. The rows
+// are known on the host, so the tiles are chosen as for a dense GEMM of 2I columns (the grouped
+// kernels' fixed 256 x 256 tiles or 16-column streaming tiles know their segments on the device
+// only). Measured (us, grouped kernels against this) at 2I x K = 10240 x 2048: 64 rows 47 / 12,
+// 2101 rows 103 / 91.
+extern "C" int sym_gemm_swiglu_bf16(const void* x, const void* w, int M, int I, int K, void* h,
+                                    void* stream) {
+  SYM_REQUIRE(M >= 0, SYM_ERR_INVALID, "gemm_swiglu_bf16: M=%d < 0", M);
+  if (M == 0) return SYM_OK;
+  SYM_REQUIRE(x && w && h, SYM_ERR_INVALID, "gemm_swiglu_bf16: null pointer argument");
+  SYM_REQUIRE(I > 0 && I % 64 == 0, SYM_ERR_UNSUPPORTED,
+              "gemm_swiglu_bf16: I=%d must be a positive multiple of 64", I);
+  SYM_REQUIRE(K > 0 && K % big::kTK == 0, SYM_ERR_UNSUPPORTED,
+              "gemm_swiglu_bf16: K=%d must be a positive multiple of %d", K, big::kTK);
+  SYM_REQUIRE((M + big::kTM - 1) / big::kTM <= 65535, SYM_ERR_UNSUPPORTED,
+              "gemm_swiglu_bf16: M=%d too large", M);
+  SYM_REQUIRE(fits_4g(M, K) && fits_4g(2ll * I, K), SYM_ERR_UNSUPPORTED,
+              "gemm_swiglu_bf16: x [%d, %d] or w [2 x %d, %d] is 4 GB or more", M, K, I, K);
+  SYM_REQUIRE(aligned(x, 16) && aligned(w, 16) && aligned(h, 16), SYM_ERR_INVALID,
+              "gemm_swiglu_bf16: x, w and h must be 16-byte aligned");
+  TileArgs p{};
+  p.a = (const uint16_t*)x;
+  p.w = (const uint16_t*)w;
+  p.M = M;
+  p.N = I;
+  p.K = K;
+  p.out_bf16 = (uint16_t*)h;
+  (void)hipGetLastError();
+  const int cus = sym_host::cu_count();
+  hipStream_t s = (hipStream_t)stream;
+  if (const DenseTiles id = dense_tiling(M, 2 * I, K, cus, false); id != kTiles256)
+    return launch_small<kGateUp>(id, p, 2 * I, s);
+  const int nx = (I + big::kTN / 2 - 1) / (big::kTN / 2);
+  hipLaunchKernelGGL(gemm_swiglu_kernel, dim3(nx, (M + big::kTM - 1) / big::kTM),
+                     dim3(big::kThreads), 0, s, p);
+  return sym_host::check_launch("gemm_swiglu_kernel");
 }
 
 // Router logits for prefill-size T on MFMA. The fp32 gate weight w [E, H] comes as three bf16

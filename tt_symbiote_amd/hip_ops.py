@@ -184,6 +184,26 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     return out
 
 
+def gemm_swiglu(x: torch.Tensor, w: torch.Tensor,
+                out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """silu(x w[:I]^T) * (x w[I:]^T) in bf16 [M, I] for x [M, K] and w [2I, K] (gate rows first)."""
+    _check(x, "x", torch.bfloat16)
+    if x.dim() != 2:
+        raise ValueError(f"x must be [M, K], got {tuple(x.shape)}")
+    M, K = x.shape
+    _check(w, "w", torch.bfloat16, x.device)
+    if w.dim() != 2 or w.shape[1] != K or w.shape[0] % 2:
+        raise ValueError(f"w must be [2I, {K}], got {tuple(w.shape)}")
+    I = w.shape[0] // 2
+    if out is None:
+        out = torch.empty(M, I, dtype=torch.bfloat16, device=x.device)
+    _check(out, "out", torch.bfloat16, x.device)
+    _check_shape(out, "out", (M, I))
+    _timed("gemm", lambda: _lib.call("sym_gemm_swiglu_bf16", _ptr(x), _ptr(w), M, I, K,
+                                     _ptr(out), _stream()))
+    return out
+
+
 def rmsnorm_linear(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor,
                    bias: Optional[torch.Tensor] = None, out_dtype: torch.dtype = torch.bfloat16,
                    out: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -209,8 +209,8 @@ def _y_dtype(weight_format: str, T: int) -> torch.dtype:
 
 
 class HIPBailingMoeV2MLP(StatelessHIPModule):
-    """Dense SwiGLU MLP (layers < first_k_dense_replace), run as one segment of the grouped
-    kernels. Replaces TTNNBailingMoeV2MLP (ttnn_moe.py; chosen at
+    """Dense SwiGLU MLP (layers < first_k_dense_replace): a gate/up product with SwiGLU and a down
+    product with the residual. Replaces TTNNBailingMoeV2MLP (ttnn_moe.py; chosen at
     modeling_bailing_moe_v2.py:388-399)."""
 
     def __init__(self):
@@ -266,6 +266,16 @@ class HIPBailingMoeV2MLP(StatelessHIPModule):
         shape = hidden_states.shape
         H = shape[-1]
         x = hidden_states.reshape(-1, H).to(torch.bfloat16).contiguous()
+        w_gate_up, w_down = self._dev["gate_up"], self._dev["down"]
+        # two dense products, their tiles chosen from the row count (which the grouped kernels
+        # know on the device only), the residual added in fp32 in the second one's epilogue: 64
+        # rows 191 -> 33 us, 2101 rows 207 -> 159 us at H = 2048, I = 5120. The grouped kernels
+        # keep the shapes these do not take as they did (H % 256, weights of 4 GB).
+        if H % 256 == 0 and 2 * w_gate_up.numel() < 1 << 32:
+            h = hip_ops.gemm_swiglu(x, w_gate_up[0])
+            res = (None if residual is None
+                   else residual.reshape(-1, H).to(torch.float32).contiguous())
+            return hip_ops.gemm(h, w_down[0], residual=res).view(shape)
         route = self._route(x.shape[0])
         _, y = hip_ops.moe_grouped_swiglu(x, route, self._dev["gate_up"], self._dev["down"],
                                           y_dtype=_y_dtype("bf16", x.shape[0]))
