@@ -19,8 +19,7 @@
 //     tile of at most 64 valid rows runs thin_tile instead: three 40 KB stages (64 A rows and
 //     256 B rows each), two steps of lookahead.
 //   gemm_small_kernel: 32 x 64 to 128 x 256 tiles for dense GEMMs of few rows (dense_tiling).
-//   gemm_tile128_kernel (router logits, N = E = 256: few tiles; grouped down projection over
-//     longer segment lists): 128 x 256 tiles, two workgroups of 8 waves per CU, each
+//   gemm_tile128_kernel (grouped down projection over longer segment lists): 128 x 256 tiles, two workgroups of 8 waves per CU, each
 //     wave a 64 x 64 block; 32 columns per step through a 3-stage 72 KB ring. The second
 //     workgroup covers a tile's prologue (segment lookup, first loads) and epilogue, which a
 //     one-workgroup shape leaves bare at 16 steps.
@@ -381,7 +380,7 @@ __device__ __forceinline__ void store_block_lds(const TileArgs& p, const floatx4
 }
 
 // ================================================================================================
-// 256 x 256 tiles (dense projections, router logits, grouped gate/up): 8 waves of 64 x 128, one
+// 256 x 256 tiles (dense projections, grouped gate/up): 8 waves of 64 x 128, one
 // workgroup per CU, 64-column steps through two 64 KB LDS stages. Per step a CU moves 64 KB from
 // L2 in whole 128-byte lines for 4 M MACs.
 // ================================================================================================
@@ -1132,7 +1131,7 @@ void gemm_f8_persistent(TileArgs p, int nx) {
 }
 
 // ================================================================================================
-// 128 x 256 tiles (grouped down projection, K = I is short; router logits, N = E is narrow): 8
+// 128 x 256 tiles (grouped down projection over long segment lists, K = I is short): 8
 // waves of 64 x 64, two workgroups per CU (while one waits at a barrier or on its prologue, the other computes), 32-column steps
 // through a 3-stage 72 KB LDS ring; a step's fragment reads are all issued before its MFMAs.
 // ================================================================================================
@@ -1444,11 +1443,12 @@ static DenseTiles dense_tiling(int M, int N, int K, int cus, bool dense) {
 
 // Small tiles of a dense product with nw weight rows (GATE_UP: 2 N).
 template <int MODE>
-static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s) {
+static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int planes = 1) {
   p.col_major = nw > p.M;
 #define SYM_LAUNCH_SMALL(TM, TN, S, WM, WN)                                                      \
   hipLaunchKernelGGL((gemm_small_kernel<MODE, TM, TN, S, WM, WN>),                               \
-                     dim3((nw + TN - 1) / TN, (p.M + TM - 1) / TM), dim3(64 * WM * WN), 0, s, p); \
+                     dim3((nw + TN - 1) / TN, (p.M + TM - 1) / TM, planes), dim3(64 * WM * WN),  \
+                     0, s, p);                                                                   \
   break
   switch (id) {
     case kTiles32x64: SYM_LAUNCH_SMALL(32, 64, 4, 2, 2);
@@ -1569,10 +1569,7 @@ extern "C" int sym_moe_router_logits_split(const void* x, const void* w_planes, 
               "moe_router_logits_split: E=%d must be a positive multiple of 16", E);
   SYM_REQUIRE(H > 0 && H % big::kTK == 0, SYM_ERR_UNSUPPORTED,
               "moe_router_logits_split: H=%d must be a positive multiple of %d", H, big::kTK);
-  // 128 x 256 tiles, two workgroups per CU: with N = E = 256 columns and three planes, 256-row
-  // tiles would leave more than half of the CUs idle at T ~ 10k
-  namespace C = mid;
-  SYM_REQUIRE((T + C::kTM - 1) / C::kTM <= 65535, SYM_ERR_UNSUPPORTED,
+  SYM_REQUIRE((T + big::kTM - 1) / big::kTM <= 65535, SYM_ERR_UNSUPPORTED,
               "moe_router_logits_split: T=%d too large", T);
   SYM_REQUIRE(fits_4g(T, H) && fits_4g(E, H), SYM_ERR_UNSUPPORTED,
               "moe_router_logits_split: x [%d, %d] is 4 GB or more", T, H);
@@ -1588,10 +1585,15 @@ extern "C" int sym_moe_router_logits_split(const void* x, const void* w_planes, 
   p.w_zstride = (long long)E * H;
   p.out_zstride = (long long)T * E;
   (void)hipGetLastError();
-  hipLaunchKernelGGL((gemm_tile128_kernel<kDense>),
-                     dim3((E + C::kTN - 1) / C::kTN, (T + C::kTM - 1) / C::kTM, 3), dim3(C::kThreads),
-                     0, (hipStream_t)stream, p);
-  return sym_host::check_launch("gemm_tile128_kernel");
+  hipStream_t s = (hipStream_t)stream;
+  // the tiles of one product with 3 E columns, one plane per grid z (E = 256, H = 2048, us,
+  // against 128 x 256 tiles of 32-column steps: 9322 tokens 48 / 35, 3431 41 / 24)
+  const DenseTiles id = dense_tiling(T, 3 * E, H, sym_host::cu_count(), false);
+  if (id != kTiles256) return launch_small<kDense>(id, p, E, s, 3);
+  hipLaunchKernelGGL((gemm_tile_kernel<kDense>),
+                     dim3((E + big::kTN - 1) / big::kTN, (T + big::kTM - 1) / big::kTM, 3),
+                     dim3(big::kThreads), 0, s, p);
+  return sym_host::check_launch("gemm_tile_kernel");
 }
 
 static int check_grouped(const char* what, int T, int H, int I, int rows, int max_segments) {
