@@ -375,6 +375,29 @@ def test_grouped_swiglu(device, T, E, H, I, top_k, skew, kernel):
         assert torch.equal(yb.cpu(), yk.bfloat16())
 
 
+@pytest.mark.parametrize("T,E,H,I,top_k", [
+    (40, 64, 256, 64, 6),      # below 12 rows per entry: thin tiles, one K-step down
+    (700, 64, 256, 64, 6),     # above 60: whole 256 x 256 tiles, one K-step down
+    (112, 64, 320, 64, 6),     # 12.06 rows per entry: 64 x 128 tiles, H and I remainders
+    (557, 64, 128, 192, 6),    # 59.99 rows per entry, two K-steps up, three down
+])
+def test_grouped_tiled_row_rule(device, T, E, H, I, top_k):
+    """Both sides of the rule that picks the grouped GEMMs' tiles, against fp32."""
+    x, wgu, wd, res = _gemm_case(T, E, H, I, top_k, seed=T, device=device, skew=True)
+    wgu, wd, x = wgu.to(device), wd.to(device), x.to(device)
+    h = torch.full((res.rows, I), float("nan"), dtype=torch.bfloat16, device=device)
+    y = torch.full((res.rows, H), float("nan"), device=device)
+    hip_ops.moe_grouped_swiglu(x, res, wgu, wd, h=h, y=y, kernel="tiled")
+    ns = int(res.n_segments.item())
+    for e, o, c in zip(*(t.cpu()[:ns].tolist()
+                         for t in (res.seg_expert, res.seg_offset, res.seg_count))):
+        xe = x[res.sorted_tokens[o:o + c].long()].float()
+        h_ref = F.silu(xe @ wgu[e, :I].float().T) * (xe @ wgu[e, I:].float().T)
+        _close(h[o:o + c], h_ref, atol=2e-3, rtol=8e-3)
+        torch.testing.assert_close(y[o:o + c], h[o:o + c].float() @ wd[e].float().T, rtol=1e-4,
+                                   atol=1e-4)
+
+
 def test_grouped_tiled_workspace_reentrant(device):
     """The tiled grouped GEMMs keep their tile counters in the caller's workspace: two streams
     running prefill-size launches at the same time, each with its own workspace, give the bytes

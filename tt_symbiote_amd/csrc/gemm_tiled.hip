@@ -744,9 +744,11 @@ void gemm_swiglu_kernel(TileArgs p) {
 // Segment list of the grouped modes in LDS (at most kPersistSeg segments): the first row tile
 // of every segment (segments past the list: the total), the estimated cost of the tiles before
 // it (kTileCost), its row count, first row and expert.
+// COST false: tiles of one height only, all taken as equal (no cpre).
 constexpr int kPersistSeg = 512;
+template <bool COST>
 struct SegTable {
-  int pre[kPersistSeg], cpre[kPersistSeg], cnt[kPersistSeg], off[kPersistSeg];
+  int pre[kPersistSeg], cpre[COST ? kPersistSeg : 1], cnt[kPersistSeg], off[kPersistSeg];
   uint16_t exp[kPersistSeg];
   int total, ctotal;
 };
@@ -766,8 +768,8 @@ __device__ __forceinline__ int row_tile_cost(int cnt, int rt, int tm) {
 
 // Wave 0 reads the segment list (all loads in flight together with n_segments; lane l owns
 // segments 8l .. 8l+7) and scans the row-tile counts of tiles of TM rows into the table.
-template <int TM, int MODE>
-__device__ __forceinline__ void load_seg_table(const TileArgs& p, SegTable& t, int nx) {
+template <int TM, int MODE, bool COST>
+__device__ __forceinline__ void load_seg_table(const TileArgs& p, SegTable<COST>& t, int nx) {
   const int lane = threadIdx.x & 63;
   if (threadIdx.x >= 64) return;
   int c[8], o[8], e[8];
@@ -803,7 +805,7 @@ __device__ __forceinline__ void load_seg_table(const TileArgs& p, SegTable& t, i
   for (int i = 0; i < 8; ++i) {
     const int sg = lane * 8 + i;
     t.pre[sg] = x - run + pre[i];
-    t.cpre[sg] = cx - crun + cpre[i];
+    if constexpr (COST) t.cpre[sg] = cx - crun + cpre[i];
     t.cnt[sg] = c[i];
     t.off[sg] = o[i];
     t.exp[sg] = (uint16_t)e[i];
@@ -817,7 +819,7 @@ __device__ __forceinline__ void load_seg_table(const TileArgs& p, SegTable& t, i
 // The first tile (index row tile * nx + column tile, in segment order) whose estimated cost
 // before it is at least c: the boundary of an XCD's run of tiles of equal cost. Wave-uniform.
 template <int TM, int MODE>
-__device__ __forceinline__ int tile_at_cost(const SegTable& t, int c, int nx) {
+__device__ __forceinline__ int tile_at_cost(const SegTable<true>& t, int c, int nx) {
   if (c <= 0) return 0;
   if (c >= t.ctotal) return t.total * nx;
   int lo = 0, hi = kPersistSeg - 1;  // the last segment whose cost prefix is <= c
@@ -835,8 +837,8 @@ __device__ __forceinline__ int tile_at_cost(const SegTable& t, int c, int nx) {
 
 // Row tile g (of TM rows) of the table: the last segment whose first row tile is <= g (binary
 // search, the same in every lane).
-template <int TM>
-__device__ __forceinline__ TileLoc seg_tile(const SegTable& t, int g, int ct) {
+template <int TM, bool COST>
+__device__ __forceinline__ TileLoc seg_tile(const SegTable<COST>& t, int g, int ct) {
   int lo = 0, hi = kPersistSeg - 1;
   while (lo < hi) {
     const int md = (lo + hi + 1) >> 1;
@@ -876,16 +878,23 @@ constexpr size_t kTicketBytes = 8 * sizeof(int);
 // the run (a ticket past the run ends the drawing workgroup); whoever reads run - 1 is the
 // last to touch the counter and resets it.
 // walk_tiles is that walk over row tiles of TM rows; tile(loc, hook) computes one tile.
-template <int TM, int MODE, typename Tile>
-__device__ __forceinline__ void walk_tiles(const TileArgs& p, int nx, SegTable& tab, int& s_next,
-                                           Tile tile) {
+template <int TM, int MODE, bool COST, typename Tile>
+__device__ __forceinline__ void walk_tiles(const TileArgs& p, int nx, SegTable<COST>& tab,
+                                           int& s_next, Tile tile) {
   load_seg_table<TM, MODE>(p, tab, nx);
   __syncthreads();
   const int x = blockIdx.x & 7, wpx = gridDim.x >> 3;
   // this XCD's tiles: the x-th eighth of the estimated cost
-  const long long ctot = tab.ctotal;
-  const int run0 = tile_at_cost<TM, MODE>(tab, (int)(ctot * x / 8), nx);
-  const int run = tile_at_cost<TM, MODE>(tab, (int)(ctot * (x + 1) / 8), nx) - run0;
+  int run0, run;
+  if constexpr (COST) {
+    const long long ctot = tab.ctotal;
+    run0 = tile_at_cost<TM, MODE>(tab, (int)(ctot * x / 8), nx);
+    run = tile_at_cost<TM, MODE>(tab, (int)(ctot * (x + 1) / 8), nx) - run0;
+  } else {
+    const long long n = (long long)__builtin_amdgcn_readfirstlane(tab.total) * nx;
+    run0 = (int)(n * x / 8);
+    run = (int)(n * (x + 1) / 8) - run0;
+  }
   // a per-lane (to the compiler: divergent) address, so the fetch-add is issued as it stands
   // and its result is waited for only where it is used
   int zero = 0;
@@ -922,7 +931,7 @@ __global__ __launch_bounds__(big::kThreads) __attribute__((amdgpu_waves_per_eu(2
 void gemm_tile_persistent(TileArgs p, int nx) {
   using namespace big;
   __shared__ __align__(1024) uint16_t smem[2 * kStage];
-  __shared__ SegTable tab;
+  __shared__ SegTable<true> tab;
   __shared__ int s_next;
   walk_tiles<kTM, MODE>(p, nx, tab, s_next, [&](const TileLoc& loc, auto hook) {
     if (loc.rows <= thin::kTM) thin_tile<MODE>(p, loc, smem, hook);
@@ -1122,7 +1131,7 @@ template <int MODE>
 __global__ __launch_bounds__(f8::kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f8_persistent(TileArgs p, int nx) {
   __shared__ __align__(1024) uint16_t smem[f8::kSmem];
-  __shared__ SegTable tab;
+  __shared__ SegTable<true> tab;
   __shared__ int s_next;
   walk_tiles<f8::kTM, MODE>(p, nx, tab, s_next, [&](const TileLoc& loc, auto hook) {
     if (loc.rows <= f8::kThinTM) f8_tile<MODE, f8::kThinTM>(p, loc, smem, hook);
@@ -1263,22 +1272,26 @@ constexpr int kTK = 64;
 constexpr int stage_elems(int tm, int tn) { return (tm + tn) * kTK; }
 }  // namespace small
 
-template <int MODE, int TM, int TN, int S, int WM = 2, int WN = 2>
-__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)))
-void gemm_small_kernel(TileArgs p) {
+// One TM x TN tile at loc. In grouped gate/up (kGather) the A rows wait for their token indices, so
+// the prologue's weight rows go first. hook() runs after the K loop, before the epilogue.
+template <int MODE, int TM, int TN, int S, int WM, int WN, bool kRagged, typename Hook>
+__device__ __forceinline__ void small_tile(TileArgs p, const TileLoc& loc, uint16_t* smem,
+                                           Hook hook) {
   using namespace small;
   constexpr int kW = WM * WN, kWR = TM / WM, kWC = TN / WN;  // waves; rows, columns of each
   constexpr int NI = kWR / 16, NJ = kWC / 16;
   constexpr int kStage = stage_elems(TM, TN), kAElems = TM * kTK;
   constexpr int kADma = TM / (8 * kW), kBDma = TN / (8 * kW), kDma = kADma + kBDma;  // per wave and step
-  __shared__ __align__(1024) uint16_t smem[S * kStage];
+  constexpr bool kGather = kRagged && MODE == kGateUp;
+  static_assert(!kRagged || (S == 3 && kADma == 1), "the wait counts");
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (opaque, as in thin_tile: per-lane values are not hoisted out of a tile loop)
+  int lane = tid & 63;
+  asm volatile("" : "+v"(lane));
   const int wm = wave / WN, wn = wave % WN;
   const int r16 = lane & 15, kq = lane >> 4;
-  TileLoc loc;
-  if (!locate_tile<kDense, TM>(p, lane, loc)) return;
-  const uint16_t* wbase = tile_weights<kDense>(p, loc);
+  const uint16_t* wbase = tile_weights<MODE>(p, loc);
 
   const int lr = lane >> 3;
   const uint32_t chunk_b = ((lane & 7) ^ lr) * 16;
@@ -1286,18 +1299,22 @@ void gemm_small_kernel(TileArgs p) {
 #pragma unroll
   for (int i = 0; i < kBDma; ++i)
     b_off[i] = b_row_offset<MODE, TN>(p, loc.ct, wave * (TN / kW) + lr + 8 * i) + chunk_b;
-#pragma unroll
-  for (int i = 0; i < kADma; ++i)
-    a_off[i] = a_row_offset<kDense>(p, loc, min(wave * (TM / kW) + lr + 8 * i, loc.rows - 1)) +
-               chunk_b;
-  auto issue = [&](int kt) {
+  // kRagged: a wave whose A rows lie past the tile's valid rows loads none, and one whose output
+  // rows do computes nothing (it still loads and syncs)
+  const bool a_on = !kRagged || wave * (TM / kW) < loc.rows;
+  const bool m_on = !kRagged || wm * kWR < loc.rows;
+  auto issue_a = [&](int kt) {
+    if (!a_on) return;
     uint16_t* st = smem + (kt % S) * kStage;
-    const uint32_t k = (uint32_t)kt * (kTK * 2);
+#pragma unroll
+    for (int i = 0; i < kADma; ++i)
+      dma16(p.a, a_off[i] + (uint32_t)kt * (kTK * 2), st + (wave * (TM / kW) + 8 * i) * kTK);
+  };
+  auto issue_b = [&](int kt) {
+    uint16_t* st = smem + (kt % S) * kStage + kAElems;
 #pragma unroll
     for (int i = 0; i < kBDma; ++i)
-      dma16(wbase, b_off[i] + k, st + kAElems + (wave * (TN / kW) + 8 * i) * kTK);
-#pragma unroll
-    for (int i = 0; i < kADma; ++i) dma16(p.a, a_off[i] + k, st + (wave * (TM / kW) + 8 * i) * kTK);
+      dma16(wbase, b_off[i] + (uint32_t)kt * (kTK * 2), st + (wave * (TN / kW) + 8 * i) * kTK);
   };
   const int sw = r16 & 7;
   const int a_frag = (wm * kWR + r16) * kTK;
@@ -1312,19 +1329,37 @@ void gemm_small_kernel(TileArgs p) {
     for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   const int nk = p.K / kTK;
+  if constexpr (kGather) {
+#pragma unroll
+    for (int i = 0; i < S - 1; ++i)
+      if (i < nk) issue_b(i);
+  }
+#pragma unroll
+  for (int i = 0; i < kADma; ++i)
+    a_off[i] = a_row_offset<MODE>(p, loc, min(wave * (TM / kW) + lr + 8 * i, loc.rows - 1)) +
+               chunk_b;
 #pragma unroll
   for (int i = 0; i < S - 1; ++i)
-    if (i < nk) issue(i);
+    if (i < nk) {
+      if constexpr (!kGather) issue_b(i);
+      issue_a(i);
+    }
   for (int kt = 0; kt < nk; ++kt) {
-    // wait for step kt; the steps issued after it stay in flight
+    // wait for step kt; the steps issued after it stay in flight (kGather, kt = 0: of step 1
+    // only its A rows were issued after step 0's)
     const int rem = min(nk - 1 - kt, S - 2);
     if (rem <= 0) SYM_TILE_SYNC_N(0);
+    else if (!a_on) SYM_TILE_SYNC_N(kBDma);
+    else if (kGather && kt == 0) SYM_TILE_SYNC_N(kADma);
     else if (rem == 1) SYM_TILE_SYNC_N(kDma);
-    else if (rem == 2) SYM_TILE_SYNC_N(2 * kDma);
-    else if (rem == 3) SYM_TILE_SYNC_N(3 * kDma);
-    else SYM_TILE_SYNC_N(4 * kDma);
+    else SYM_TILE_SYNC_N(2 * kDma);
+    static_assert(S <= 4, "the wait counts");
     // the barrier also means that every wave has read the stage refilled here
-    if (kt + S - 1 < nk) issue(kt + S - 1);
+    if (kt + S - 1 < nk) {
+      issue_b(kt + S - 1);
+      issue_a(kt + S - 1);
+    }
+    if (!m_on) continue;
     const uint16_t* st = smem + (kt % S) * kStage;
     u32x4 a[2][NI], b[2][NJ];
 #pragma unroll
@@ -1347,8 +1382,37 @@ void gemm_small_kernel(TileArgs p) {
               __builtin_bit_cast(bf16x8, b[h][j]), __builtin_bit_cast(bf16x8, a[h][i]),
               acc[i][j], 0, 0, 0);
   }
+  hook();
   const int col0 = MODE == kGateUp ? loc.ct * (TN / 2) + wn * (kWC / 2) : loc.ct * TN + wn * kWC;
   store_block<MODE>(p, acc, loc, wm * kWR, col0, lane);
+}
+
+template <int MODE, int TM, int TN, int S, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_small_kernel(TileArgs p) {
+  __shared__ __align__(1024) uint16_t smem[S * small::stage_elems(TM, TN)];
+  TileLoc loc;
+  if (!locate_tile<kDense, TM>(p, threadIdx.x & 63, loc)) return;
+  small_tile<MODE, TM, TN, S, WM, WN, false>(p, loc, smem, NoHook{});
+}
+
+// The grouped expert GEMMs on 64 x 128 tiles, two workgroups of 8 waves per CU, over the persistent
+// walk: for segment lists whose experts have few rows each, where streaming the weights is the
+// bound. Against the 256 x 256 kernel's thin tiles (one workgroup per CU): a tile is half as long,
+// so the last round leaves less of the chip idle (257 experts are 4.02 rounds of thin gate/up
+// tiles per CU, in practice 5), and one workgroup's prologue and epilogue run under the other's
+// loads.
+constexpr int kNarrowTM = 64, kNarrowTN = 128, kNarrowS = 3;
+template <int MODE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
+void gemm_narrow_persistent(TileArgs p, int nx) {
+  __shared__ __align__(1024) uint16_t smem[kNarrowS * small::stage_elems(kNarrowTM, kNarrowTN)];
+  __shared__ SegTable<false> tab;
+  __shared__ int s_next;
+  static_assert(sizeof(smem) + sizeof(tab) + 16 <= 80 * 1024, "two workgroups per CU");
+  walk_tiles<kNarrowTM, MODE>(p, nx, tab, s_next, [&](const TileLoc& loc, auto hook) {
+    small_tile<MODE, kNarrowTM, kNarrowTN, kNarrowS, 2, 4, true>(p, loc, smem, hook);
+  });
 }
 
 }  // namespace sym
@@ -1624,6 +1688,15 @@ static int check_tickets(const char* what, const void* workspace, size_t workspa
   return SYM_OK;
 }
 
+// Which grouped launches take 64 x 128 tiles: those with 12 to 60 rows per list entry. gate/up +
+// down of 257 experts of 512 x 2048 (us, 256 x 256 against 64 x 128 tiles, even / Zipf load):
+// 333 tokens (12 rows) 313 / 301 against 317 / 300, 640 tokens 328 / 333 against 316 / 336, 900
+// tokens 340 / 355 against 325 / 340, 1200 tokens 348 / 373 against 335 / 351, 1600 tokens (56
+// rows) 361 / 383 against 350 / 382, 2048 tokens (72 rows) 390 / 410 against 413 / 413.
+static bool narrow_tiles(int rows, int max_segments) {
+  return max_segments <= kPersistSeg && rows >= 12ll * max_segments && rows <= 60ll * max_segments;
+}
+
 extern "C" size_t sym_moe_tiled_workspace_bytes(void) { return kTicketBytes; }
 
 extern "C" int sym_moe_gate_up_tiled(const void* x, int T, int H, int I, int rows,
@@ -1656,6 +1729,12 @@ extern "C" int sym_moe_gate_up_tiled(const void* x, int T, int H, int I, int row
   p.tickets = (int*)workspace;
   (void)hipGetLastError();
   namespace C = big;
+  if (narrow_tiles(rows, max_segments)) {
+    const int grid = std::max(8, sym_host::cu_count() / 8 * 8) * 2;  // two workgroups per CU
+    hipLaunchKernelGGL((gemm_narrow_persistent<kGateUp>), dim3(grid), dim3(512), 0,
+                       (hipStream_t)stream, p, (I + kNarrowTN / 2 - 1) / (kNarrowTN / 2));
+    return sym_host::check_launch("gemm_narrow_persistent");
+  }
   const int nx = (I + C::kTN / 2 - 1) / (C::kTN / 2);
   if (max_segments <= kPersistSeg) {
     // one workgroup per CU, a multiple of 8 (one run of tiles per XCD)
@@ -1696,6 +1775,12 @@ extern "C" int sym_moe_down_tiled(const void* h, int T, int H, int I, int rows,
   else p.out_f32 = (float*)y;
   p.tickets = (int*)workspace;
   (void)hipGetLastError();
+  if (narrow_tiles(rows, max_segments)) {
+    const int grid = std::max(8, sym_host::cu_count() / 8 * 8) * 2;  // two workgroups per CU
+    hipLaunchKernelGGL((gemm_narrow_persistent<kDown>), dim3(grid), dim3(512), 0,
+                       (hipStream_t)stream, p, (H + kNarrowTN - 1) / kNarrowTN);
+    return sym_host::check_launch("gemm_narrow_persistent");
+  }
   if (max_segments <= kPersistSeg) {
     const int grid = std::max(8, sym_host::cu_count() / 8 * 8);
     hipLaunchKernelGGL((gemm_tile_persistent<kDown>), dim3(grid), dim3(big::kThreads), 0,
