@@ -138,6 +138,14 @@ def test_route_permute_bit_exact(device, T, E, n_group, topk_group, top_k, kind,
         assert np.array_equal(getattr(res, name).cpu().numpy()[:ns], p[name][:ns]), name
 
 
+@pytest.mark.parametrize("T", [1, 5, 12, 13, 64, 65])
+@pytest.mark.parametrize("E,top_k", [(64, 32), (256, 8)])
+def test_route_permute_batch_edges(device, T, E, top_k):
+    """Both sides of the one-launch limit (12 tokens) and of a mask word (64), with the largest
+    top_k."""
+    test_route_permute_bit_exact(device, T, E, 1, 1, top_k, "zipf", True)
+
+
 def test_route_no_renorm(device):
     logits, bias = _route_inputs(40, 256, "randn", seed=3)
     kw = dict(n_group=8, topk_group=4, top_k=8, routed_scale=2.5, renormalize=False)

@@ -338,6 +338,88 @@ __global__ __launch_bounds__(kPermuteThreads) void moe_permute_kernel(
   }
 }
 
+// Route and permute of a decode batch of at most kFusedTokens tokens in one launch (one workgroup,
+// wave w routing token w), the same outputs as the two kernels above, bit for bit. Both are bound
+// by latency: the routing of a token is a chain of dependent lane operations, the permute one of
+// LDS steps, and the second launch costs as much as either (us in a replayed graph, two launches
+// against one: 1 token 6.9 / 5.4, 4 7.4 / 5.8, 8 7.7 / 6.3, 12 7.9 / 7.1). More tokens share the one
+// workgroup's SIMDs and lose it again (16: 7.9 / 8.1, 32: 8.0 / 12.6). With at most 64 tokens one
+// mask word per expert holds them all; its popcount is the expert's count, and the scans of counts
+// and of used experts share one (a count is below 2^16).
+constexpr int kFusedTokens = 12;
+template <int EPL>
+__global__ __launch_bounds__(kPermuteThreads) void moe_route_permute_kernel(
+    const float* __restrict__ logits, int n_parts, const float* __restrict__ bias, int T, int E,
+    int n_group, int topk_group, int top_k, float routed_scale, int renorm, int with_shared,
+    int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
+    int32_t* __restrict__ expert_counts, int32_t* __restrict__ expert_offsets,
+    int32_t* __restrict__ sorted_tokens, int32_t* __restrict__ inv_perm,
+    int32_t* __restrict__ seg_expert, int32_t* __restrict__ seg_offset,
+    int32_t* __restrict__ seg_count, int32_t* __restrict__ n_segments) {
+  constexpr int kWaves = kPermuteThreads / 64;
+  static_assert(kFusedTokens <= kWaves, "a wave per token");
+  __shared__ unsigned long long s_mask[64 * EPL];
+  __shared__ int s_off[64 * EPL];
+  __shared__ int s_idx[kFusedTokens * kMaxTopK];
+  __shared__ int s_wave[kWaves];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int TK = T * top_k;
+  float parts[kLogitParts][EPL], bv[EPL];
+  const int t = wave;
+  // (a wave without a token repeats the last one's loads)
+  load_token_logits<EPL>(logits, n_parts, (size_t)T * E, min(t, T - 1), E, lane, parts);
+#pragma unroll
+  for (int j = 0; j < EPL; ++j) bv[j] = bias[lane * EPL + j];
+  if (tid < E) s_mask[tid] = 0ull;
+  __syncthreads();
+  if (t < T) {
+    int my_idx;
+    float my_w;
+    route_token<EPL>(parts, n_parts, bv, E, n_group, topk_group, top_k, routed_scale, renorm, lane,
+                     my_idx, my_w);
+    if (lane < top_k) {
+      topk_idx[t * top_k + lane] = my_idx;
+      topk_w[t * top_k + lane] = my_w;
+      s_idx[t * top_k + lane] = my_idx;
+      atomicOr(&s_mask[my_idx], 1ull << t);
+    }
+  }
+  __syncthreads();
+  const int e = tid;
+  const int cnt = e < E ? __popcll(s_mask[e]) : 0;
+  int total = 0;
+  const int pre = block_exclusive_scan(cnt | (cnt > 0 ? 1 << 16 : 0), s_wave, &total);
+  const int off = pre & 0xffff, slot = pre >> 16, n_routed = total >> 16;
+  if (e < E) {
+    s_off[e] = off;
+    expert_counts[e] = cnt;
+    expert_offsets[e] = off;
+    if (cnt > 0) {
+      seg_expert[slot] = e;
+      seg_offset[slot] = off;
+      seg_count[slot] = cnt;
+    }
+  }
+  if (tid == 0) {
+    expert_offsets[E] = total & 0xffff;
+    if (with_shared) {
+      seg_expert[n_routed] = E;
+      seg_offset[n_routed] = TK;
+      seg_count[n_routed] = T;
+    }
+    n_segments[0] = n_routed + (with_shared ? 1 : 0);
+  }
+  if (with_shared && tid < T) sorted_tokens[TK + tid] = tid;
+  __syncthreads();
+  for (int a = tid; a < TK; a += kPermuteThreads) {
+    const int ta = a / top_k, ex = s_idx[a];
+    const int row = s_off[ex] + __popcll(s_mask[ex] & ((1ull << ta) - 1ull));
+    sorted_tokens[row] = ta;
+    inv_perm[a] = row;
+  }
+}
+
 // Permute of many tokens across the GPU (the same outputs as moe_permute_kernel, bit for bit),
 // in three launches over chunks of kChunkTokens tokens:
 //   1. moe_permute_count_kernel: per (chunk, expert) assignment counts (LDS atomics);
@@ -731,6 +813,21 @@ extern "C" int sym_moe_route_permute(const float* logits, int n_logit_parts, con
 
   hipStream_t s = (hipStream_t)stream;
   (void)hipGetLastError();
+  if (T <= kFusedTokens) {
+#define SYM_LAUNCH_ROUTE_PERMUTE(EE)                                                             \
+  hipLaunchKernelGGL(moe_route_permute_kernel<EE>, dim3(1), dim3(kPermuteThreads), 0, s, logits,  \
+                     n_logit_parts, bias, T, E, n_group, topk_group, top_k, routed_scale,         \
+                     renormalize, with_shared, topk_idx, topk_w, expert_counts, expert_offsets,   \
+                     sorted_tokens, inv_perm, seg_expert, seg_offset, seg_count, n_segments)
+    switch (epl) {
+      case 1: SYM_LAUNCH_ROUTE_PERMUTE(1); break;
+      case 2: SYM_LAUNCH_ROUTE_PERMUTE(2); break;
+      case 4: SYM_LAUNCH_ROUTE_PERMUTE(4); break;
+      default: SYM_LAUNCH_ROUTE_PERMUTE(8); break;
+    }
+#undef SYM_LAUNCH_ROUTE_PERMUTE
+    return sym_host::check_launch("moe_route_permute_kernel");
+  }
   const dim3 grid((T + 3) / 4), block(256);
 #define SYM_LAUNCH_ROUTE(EE)                                                                    \
   hipLaunchKernelGGL(moe_route_kernel<EE>, grid, block, 0, s, logits, n_logit_parts, bias, T, E, \
