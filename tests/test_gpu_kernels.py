@@ -489,7 +489,8 @@ def test_gemm_tiled(device, M, N, K, bias, res, out_dtype):
     (1, 16, 64), (31, 3072, 2048), (33, 2048, 128),       # 32 x 64 tiles, one or two K-steps
     (65, 4096, 192), (300, 3072, 256), (512, 3056, 320),  # 64 x 64
     (1000, 2064, 256), (900, 2048, 448),                  # 64 x 128
-    (1500, 3072, 64), (2101, 2048, 5120), (5400, 3088, 128),  # 128 x 128
+    (1500, 3072, 64), (2101, 2048, 5120),                 # 96 x 128
+    (3431, 2048, 192), (5400, 3088, 128),                 # 128 x 128
     (17, 131200, 1024), (50, 131216, 1024), (129, 131088, 1088),  # weights over 256 MB
 ])
 @pytest.mark.parametrize("kind", ["bf16", "f32", "bias_res32", "res16"])

@@ -1471,9 +1471,11 @@ static void dense_tail_split(int M, int nx, int cus, int& full_rt, int& tail_row
 // further one on the busiest CU `more`, with the load halfway between the mean and the busiest
 // CU's (fitted to sweeps of M = 16 .. 9322 at N = 2048 and 3072, K = 2048 and 5120; time scales
 // with K). Measured (us, 256 x 256 against the choice) for N x K = 3072 x 2048: M = 64 27.6 /
-// 10.0, 333 32.2 / 13.9, 512 31.8 / 14.7, 1024 33.4 / 22.1, 1710 33.8 / 32.3; 256 x 256 stays for
+// 10.0, 333 32.2 / 13.9, 512 31.8 / 14.7, 1024 33.4 / 22.1, 1710 33.8 / 26.7; 256 x 256 stays for
 // 2560-5000 (46.2 / 54.9 at 3431) and from 5600 rows (101.5 / 120.5 at 9322).
-enum DenseTiles { kTiles32x64, kTiles64x64, kTiles64x128, kTiles128x128, kTiles128x256, kTiles256 };
+enum DenseTiles {
+  kTiles32x64, kTiles64x64, kTiles64x128, kTiles96x128, kTiles128x128, kTiles128x256, kTiles256
+};
 static DenseTiles dense_tiling(int M, int N, int K, int cus, bool dense) {
   if (dense && (long long)N * K * 2 > (256ll << 20) && M <= 256)
     return M <= 32 ? kTiles32x64 : M <= 64 ? kTiles64x128 : kTiles128x256;
@@ -1485,6 +1487,7 @@ static DenseTiles dense_tiling(int M, int N, int K, int cus, bool dense) {
   static const Kind kinds[] = {{kTiles32x64, 32, 64, 10.0, 4.4},
                                {kTiles64x64, 64, 64, 11.0, 6.5},
                                {kTiles64x128, 64, 128, 15.0, 9.0},
+                               {kTiles96x128, 96, 128, 18.0, 13.0},
                                {kTiles128x128, 128, 128, 20.0, 16.5}};
   const long long big_tiles = (long long)((M + 255) / 256) * ((N + 255) / 256);
   double best = big_tiles <= cus ? 30.0 + 16.0 * big_tiles / cus
@@ -1518,6 +1521,7 @@ static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int p
     case kTiles32x64: SYM_LAUNCH_SMALL(32, 64, 4, 2, 2);
     case kTiles64x64: SYM_LAUNCH_SMALL(64, 64, 3, 2, 2);
     case kTiles64x128: SYM_LAUNCH_SMALL(64, 128, 3, 2, 4);
+    case kTiles96x128: SYM_LAUNCH_SMALL(96, 128, 2, 2, 2);
     case kTiles128x128: SYM_LAUNCH_SMALL(128, 128, 2, 2, 4);
     default: SYM_LAUNCH_SMALL(128, 256, 3, 2, 4);
   }
@@ -1585,7 +1589,7 @@ extern "C" int sym_gemm_bf16_res_bf16(const void* a, const void* w, const void* 
 // are known on the host, so the tiles are chosen as for a dense GEMM of 2I columns (the grouped
 // kernels' fixed 256 x 256 tiles or 16-column streaming tiles know their segments on the device
 // only). Measured (us, grouped kernels against this) at 2I x K = 10240 x 2048: 64 rows 47 / 12,
-// 2101 rows 103 / 91.
+// 2101 rows 103 / 92.
 extern "C" int sym_gemm_swiglu_bf16(const void* x, const void* w, int M, int I, int K, void* h,
                                     void* stream) {
   SYM_REQUIRE(M >= 0, SYM_ERR_INVALID, "gemm_swiglu_bf16: M=%d < 0", M);
