@@ -102,6 +102,7 @@ def test_grouped_swiglu_fp8_tiled(device, monkeypatch, T, E, H, I, top_k, hot):
                                     with_shared=True)
     hs, ys = hip_ops.moe_grouped_swiglu(x, res, *q, kernel="stream")
     monkeypatch.setattr(hip_ops, "TILED_MIN_TOKENS_FP8", 1)
+    monkeypatch.setattr(hip_ops, "TILED_MIN_TOKENS_FP8_DOWN", 1)
     h = torch.full_like(hs, float("nan"))
     y = torch.full_like(ys, float("nan"))
     hip_ops.moe_grouped_swiglu(x, res, *q, h=h, y=y)

@@ -874,10 +874,14 @@ def moe_route_permute(logits: torch.Tensor, bias: torch.Tensor, *, n_group: int,
 
 TILED_MIN_TOKENS = 128  # from this many tokens the expert GEMMs use the tiled (MFMA-bound) kernels
 
-# The same for fp8 expert weights (gate/up + down of 257 segments of 512 x 2048, us, streaming
-# against tiled): 192 tokens 158 / 194 (even load), 180 / 180 (Zipf); 256: 173 / 200, 205 / 197;
-# 320: 194 / 205, 259 / 200; 512: 264 / 221, 318 / 230; 3431 (Zipf): 1847 / 401.
+# The same for fp8 expert weights, gate/up and down apart: the streaming down kernel keeps its
+# weights in registers for all 16-row passes, the gate/up kernel re-reads them. 257 segments of 512
+# x 2048, us, streaming against tiled, even / Zipf load: gate/up 128 tokens 98 / 95 against 118 /
+# 112, 256: 123 / 180 against 127 / 119, 512: 203 / 290 against 139 / 142; down 256: 54 / 56 against
+# 74 / 71, 640: 73 / 76 against 83 / 84, 1024: 102 / 105 against 92 / 95, 2048: 184 / 187 against
+# 126 / 125.
 TILED_MIN_TOKENS_FP8 = 256
+TILED_MIN_TOKENS_FP8_DOWN = 832
 
 
 def moe_tiled_workspace(device=None) -> torch.Tensor:
@@ -991,30 +995,34 @@ def moe_grouped_swiglu(x: torch.Tensor, route: RouteResult, w_gate_up,
     if fp8:
         if kernel == "tiled":
             raise NotImplementedError("fp8 expert weights: only \"auto\" picks the tiled kernels")
-        # the tiled kernels' limits: one weight tile is 256 rows, 32-bit byte offsets
-        if (kernel == "auto" and T >= TILED_MIN_TOKENS_FP8 and max_segments <= 512
-                and max(2 * T * H, 2 * rows * I, 4 * I * H) < 1 << 32
-                and rows // 128 + max_segments <= 65535):
-            ws = moe_tiled_workspace(dev)
+        # the tiled kernels' limits: the segment list in LDS, 32-bit byte offsets
+        fits = (max_segments <= 512 and max(2 * T * H, 2 * rows * I, 4 * I * H) < 1 << 32
+                and rows // 128 + max_segments <= 65535)
+        up_tiled = kernel == "auto" and fits and T >= TILED_MIN_TOKENS_FP8
+        down_tiled = kernel == "auto" and fits and T >= TILED_MIN_TOKENS_FP8_DOWN
+        ws = moe_tiled_workspace(dev) if up_tiled or down_tiled else None
+        if up_tiled:
             _timed("moe_gate_up", lambda: _lib.call(
                 "sym_moe_gate_up_fp8_tiled", _ptr(x), T, H, I, rows, _ptr(route.sorted_tokens),
                 _ptr(route.seg_expert), _ptr(route.seg_offset), _ptr(route.seg_count),
                 _ptr(route.n_segments), max_segments, _ptr(w_gate_up), _ptr(s_gate_up), _ptr(h),
                 _ptr(ws), ws.numel(), stream))
+        else:
+            _timed("moe_gate_up", lambda: _lib.call(
+                "sym_moe_gate_up_fp8", _ptr(x), T, H, I, _ptr(route.sorted_tokens),
+                _ptr(route.seg_expert), _ptr(route.seg_offset), _ptr(route.seg_count),
+                _ptr(route.n_segments), max_segments, _ptr(w_gate_up), _ptr(s_gate_up), _ptr(h),
+                stream))
+        if down_tiled:
             _timed("moe_down", lambda: _lib.call(
                 "sym_moe_down_fp8_tiled", _ptr(h), T, H, I, rows, _ptr(route.seg_expert),
                 _ptr(route.seg_offset), _ptr(route.seg_count), _ptr(route.n_segments),
                 max_segments, _ptr(w_down), _ptr(s_down), _ptr(y), _ptr(ws), ws.numel(), stream))
-            return h, y
-        _timed("moe_gate_up", lambda: _lib.call(
-            "sym_moe_gate_up_fp8", _ptr(x), T, H, I, _ptr(route.sorted_tokens),
-            _ptr(route.seg_expert), _ptr(route.seg_offset), _ptr(route.seg_count),
-            _ptr(route.n_segments), max_segments, _ptr(w_gate_up), _ptr(s_gate_up), _ptr(h),
-            stream))
-        _timed("moe_down", lambda: _lib.call(
-            "sym_moe_down_fp8", _ptr(h), T, H, I, _ptr(route.seg_expert), _ptr(route.seg_offset),
-            _ptr(route.seg_count), _ptr(route.n_segments), max_segments, _ptr(w_down),
-            _ptr(s_down), _ptr(y), stream))
+        else:
+            _timed("moe_down", lambda: _lib.call(
+                "sym_moe_down_fp8", _ptr(h), T, H, I, _ptr(route.seg_expert),
+                _ptr(route.seg_offset), _ptr(route.seg_count), _ptr(route.n_segments),
+                max_segments, _ptr(w_down), _ptr(s_down), _ptr(y), stream))
         return h, y
     if tiled:
         if workspace is None:
