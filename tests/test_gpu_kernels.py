@@ -870,6 +870,43 @@ def test_prefill_prologue_matches_decode_prologue(device):
     assert torch.equal(v.cpu(), qkv.cpu().view(T, Hq + 2 * Hkv, D)[:, Hq + Hkv:])
 
 
+@pytest.mark.parametrize("Hq,Hkv,rd,norm", [
+    (16, 4, 64, True), (32, 8, 128, True),   # one and two rounds of 24 heads
+    (4, 1, 16, True), (5, 5, 0, True), (16, 2, 64, False),
+    (8, 2, 24, True),                        # rd % 16 != 0: one wave per head
+])
+def test_prefill_prologue_forms(device, Hq, Hkv, rd, norm):
+    """Bit for bit the decode prologue over head counts, rotary widths and positions outside the
+    table (kept unrotated) or the page table (not written), T not a multiple of 4 tokens."""
+    T, D, bs, nb, max_pos = 67, 128, 16, 9, 100
+    g = torch.Generator(device=device).manual_seed(Hq + rd)
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, generator=g, device=device).bfloat16()
+    pos = torch.arange(T, dtype=torch.int32, device=device) * 2
+    pos[3], pos[T - 1] = -1, 4000
+    sid = torch.zeros(T, dtype=torch.int32, device=device)
+    pt = torch.randperm(nb, generator=g, device=device)[None].int().contiguous()
+    w = (1 + 0.1 * torch.randn(2, D, generator=g, device=device)).bfloat16()
+    kw = dict(num_heads=Hq, num_kv_heads=Hkv, rotary_dim=rd, eps=1e-6,
+              rope_cs=torch.randn(max_pos, rd, generator=g, device=device) if rd else None,
+              q_norm_w=w[0].contiguous() if norm else None,
+              k_norm_w=w[1].contiguous() if norm else None)
+    pools = [torch.zeros(nb, Hkv, bs, D, dtype=torch.bfloat16, device=device) for _ in range(4)]
+    q, k, v = hip_ops.attn_prefill_prologue(qkv, pos, sid, pools[0], pools[1], pt, **kw)
+    q2 = hip_ops.attn_decode_prologue(qkv, pos, pools[2], pools[3],
+                                      pt.expand(T, -1).contiguous(), **kw)
+    assert torch.equal(q, q2)
+    assert torch.equal(pools[0], pools[2]) and torch.equal(pools[1], pools[3])
+    slots = [t for t in range(T) if 0 <= int(pos[t]) < nb * bs]
+    for t in slots:
+        p = int(pos[t])
+        assert torch.equal(k[t], pools[2][int(pt[0, p // bs]), :, p % bs])
+    assert torch.equal(v, qkv.view(T, Hq + 2 * Hkv, D)[:, Hq + Hkv:])
+    # without the pools (an fp8 cache) the same q, k and v
+    fp8 = torch.zeros(nb, Hkv, bs, D, device=device).to(torch.float8_e4m3fn)
+    for a, b in zip((q, k, v), hip_ops.attn_prefill_prologue(qkv, pos, sid, fp8, fp8, pt, **kw)):
+        assert torch.equal(a, b)
+
+
 def test_hbm_read_probe(device):
     # measurement kernel: must read every byte (a rate above the 8 TB/s HBM peak would mean
     # skipped work) and launch cleanly
