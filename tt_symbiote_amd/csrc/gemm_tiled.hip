@@ -74,6 +74,7 @@ struct TileArgs {
   int full_rt;              // DENSE with tail_rows > 0: row tiles 0 .. full_rt - 1 have TM rows,
   int tail_rows;            // the rows from full_rt * TM on tiles of tail_rows (one plane)
   int col_major;            // DENSE: the row tiles of a column tile are neighbours (N > M)
+  int rotate_k;             // K-steps start at the column tile's index (KOrder)
   int* tickets;             // persistent grids: the caller's 8 per-XCD tile counters
   const float* w_scale;     // fp8 weights: [S, rows / 128, K / 128] block scales
 };
@@ -202,6 +203,26 @@ __device__ __forceinline__ bool locate_tile(const TileArgs& p, int lane, TileLoc
     }
     return found;  // (always true: g < ntile)
   }
+}
+
+// K-steps of a tile in the order first, first + 1, .., nk - 1, 0, .., first - 1 (the sums are taken
+// in that order). Rows of the operands are a power of two apart, so workgroups that walk the same
+// K-steps at the same time ask the same few L2 channels and HBM banks for all of their rows; a
+// first step that differs from column tile to column tile spreads them. Used where it measured
+// faster: dense products whose weights stream from HBM (96 x 157184 x 2048 169 -> 149 us, 64 rows
+// 143 -> 136) and the fp8 expert products (3431 tokens, Zipf load: gate/up 238 -> 235 us, down 170
+// -> 165). Dense products that hit in L2 gain nothing and lose some of the sharing between
+// neighbouring tiles (3072 x 2048 at 9322 rows 99 -> 102 us); the bf16 expert products gain nothing
+// at 9322 tokens and lose 2% at 333.
+struct KOrder {
+  int first, nk;
+  __device__ __forceinline__ int operator()(int kt) const {
+    const int k = kt + first;
+    return k >= nk ? k - nk : k;
+  }
+};
+__device__ __forceinline__ KOrder k_order(const TileLoc& loc, int nk, bool rotate) {
+  return KOrder{rotate ? loc.ct % nk : 0, nk};
 }
 
 // Output-plane and weight-matrix bases of a tile: DENSE plane z; GATE_UP / DOWN expert e.
@@ -417,6 +438,7 @@ __device__ __forceinline__ void big_tile(TileArgs p, const TileLoc& loc, uint16_
   const int K = p.K;
 
   const uint16_t* wbase = tile_weights<MODE>(p, loc);
+  const int nk = K / kTK;
 
   // ---- LDS-DMA sources: this wave fills A rows kARows w .. and B rows kBRows w .. of every
   // stage; lane l takes row + l / 8, slot l % 8, i.e. global chunk slot ^ swz(row). A rows at
@@ -510,7 +532,6 @@ __device__ __forceinline__ void big_tile(TileArgs p, const TileLoc& loc, uint16_
   // run while half 1's fragments are read; then wait for step kt + 1's stage and barrier (every
   // wave has read all of step kt, so its stage is free), issue step kt + 2 into it, and run the
   // MFMAs of half 1 while half 0 of step kt + 1 is read.
-  const int nk = K / kTK;
   auto stage_of = [&](int kt) { return smem + (kt & 1) * kStage; };
   auto loop = [&](auto ni_tag) {
     constexpr bool kMfma = decltype(ni_tag)::value > 0;
@@ -604,6 +625,7 @@ __device__ __forceinline__ void thin_tile(TileArgs p, const TileLoc& loc, uint16
   const int wn = wave % kWavesN;
   const int r16 = lane & 15, kq = lane >> 4;
   const uint16_t* wbase = tile_weights<MODE>(p, loc);
+  const int nk = p.K / kTK;
 
   // DMA: wave w fills A rows 8w .. 8w + 7 (while the tile has rows there) and B rows 32w ..
   // 32w + 31 of each stage, lane l taking row + l / 8, chunk slot (l % 8) ^ swz(row)
@@ -626,7 +648,6 @@ __device__ __forceinline__ void thin_tile(TileArgs p, const TileLoc& loc, uint16
 #pragma unroll
     for (int i = 0; i < kBDma; ++i) dma16(wbase, b_off[i] + k, stage_of(kt) + b_dst + i * 512);
   };
-  const int nk = p.K / kTK;
   // wait for step kt, leaving what was issued after it in flight: at kt = 0 (issued B0, B1,
   // A0, A1) step 1's A instruction, or for a wave without A rows step 1's 4 B instructions;
   // later, step kt + 1's 5 (or 4) instructions, issued after all of step kt
@@ -984,6 +1005,8 @@ __device__ __forceinline__ void f8_tile(const TileArgs& p, const TileLoc& loc, u
   const int wm = wave / WN, wn = wave % WN;
   const int r16 = lane & 15, kq = lane >> 4;
   const int K = p.K, nk = K / kTK;
+  // (the scales are held 64 steps at a time, in step order)
+  const KOrder kk_of = k_order(loc, nk, p.rotate_k && nk <= 64);
   const int wrows = MODE == kGateUp ? 2 * p.N : p.N;  // weight rows of one expert
   const uint16_t* wbase =
       reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(p.w) +
@@ -1010,7 +1033,7 @@ __device__ __forceinline__ void f8_tile(const TileArgs& p, const TileLoc& loc, u
   auto issue_b = [&](int kt) {
     uint16_t* st = stage_of(kt) + kAElems + wave * 32 * 64;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma16(wbase, b_off[i] + (uint32_t)kt * kTK, st + i * 512);
+    for (int i = 0; i < 4; ++i) dma16(wbase, b_off[i] + (uint32_t)kk_of(kt) * kTK, st + i * 512);
   };
   auto issue_a = [&](int kt) {
     if (!a_on) return;
@@ -1019,7 +1042,7 @@ __device__ __forceinline__ void f8_tile(const TileArgs& p, const TileLoc& loc, u
     for (int i = 0; i < kAInst; ++i)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        dma16(p.a, a_off[i] + (uint32_t)kt * (2 * kTK) + h * 128, st + h * (TM * 64) + i * 512);
+        dma16(p.a, a_off[i] + (uint32_t)kk_of(kt) * (2 * kTK) + h * 128, st + h * (TM * 64) + i * 512);
   };
   auto rows_of_a = [&]() {
 #pragma unroll
@@ -1084,9 +1107,9 @@ __device__ __forceinline__ void f8_tile(const TileArgs& p, const TileLoc& loc, u
                                                        i * 16 * 64 +
                                                        ((2 * kq + (kk & 1)) ^ sw) * 8);
         const float c0 = __builtin_bit_cast(
-            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sv0), kt & 63));
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sv0), kk_of(kt) & 63));
         const float c1 = __builtin_bit_cast(
-            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sv1), kt & 63));
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sv1), kk_of(kt) & 63));
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           uint4 b[4];
@@ -1303,18 +1326,20 @@ __device__ __forceinline__ void small_tile(TileArgs p, const TileLoc& loc, uint1
   // rows do computes nothing (it still loads and syncs)
   const bool a_on = !kRagged || wave * (TM / kW) < loc.rows;
   const bool m_on = !kRagged || wm * kWR < loc.rows;
+  const int nk = p.K / kTK;
+  const KOrder kk_of = k_order(loc, nk, !kRagged && p.rotate_k);
   auto issue_a = [&](int kt) {
     if (!a_on) return;
     uint16_t* st = smem + (kt % S) * kStage;
 #pragma unroll
     for (int i = 0; i < kADma; ++i)
-      dma16(p.a, a_off[i] + (uint32_t)kt * (kTK * 2), st + (wave * (TM / kW) + 8 * i) * kTK);
+      dma16(p.a, a_off[i] + (uint32_t)kk_of(kt) * (kTK * 2), st + (wave * (TM / kW) + 8 * i) * kTK);
   };
   auto issue_b = [&](int kt) {
     uint16_t* st = smem + (kt % S) * kStage + kAElems;
 #pragma unroll
     for (int i = 0; i < kBDma; ++i)
-      dma16(wbase, b_off[i] + (uint32_t)kt * (kTK * 2), st + (wave * (TN / kW) + 8 * i) * kTK);
+      dma16(wbase, b_off[i] + (uint32_t)kk_of(kt) * (kTK * 2), st + (wave * (TN / kW) + 8 * i) * kTK);
   };
   const int sw = r16 & 7;
   const int a_frag = (wm * kWR + r16) * kTK;
@@ -1328,7 +1353,6 @@ __device__ __forceinline__ void small_tile(TileArgs p, const TileLoc& loc, uint1
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  const int nk = p.K / kTK;
   if constexpr (kGather) {
 #pragma unroll
     for (int i = 0; i < S - 1; ++i)
@@ -1463,21 +1487,22 @@ static void dense_tail_split(int M, int nx, int cus, int& full_rt, int& tail_row
 }
 
 // Which tiles a dense GEMM runs on.
-// A weight too large for the caches (over 256 MB, e.g. an LM head) streams from HBM whatever the
+// A weight too large for the caches (over kCacheBytes, e.g. an LM head) streams from HBM whatever the
 // tile, so the one with the fewest operand re-reads that covers M is taken (157184 x 2048, us,
-// 256 x 256 tiles against the choice): 32 rows 161 / 126 on 32 x 64; 64: 176 / 135 on 64 x 128;
-// 96: 189 / 160, 128: 198 / 168, 256: 272 / 214 on 128 x 256 (16: 154 / 119).
+// 256 x 256 tiles against the choice): 32 rows 161 / 126 on 32 x 64; 64: 176 / 136 on 64 x 128;
+// 96: 189 / 149, 128: 198 / 168, 256: 272 / 209 on 128 x 256 (16: 154 / 119).
 // Otherwise by estimated time: at K = 2048 a workgroup alone on its CU takes `alone` us and each
 // further one on the busiest CU `more`, with the load halfway between the mean and the busiest
 // CU's (fitted to sweeps of M = 16 .. 9322 at N = 2048 and 3072, K = 2048 and 5120; time scales
 // with K). Measured (us, 256 x 256 against the choice) for N x K = 3072 x 2048: M = 64 27.6 /
 // 10.0, 333 32.2 / 13.9, 512 31.8 / 14.7, 1024 33.4 / 22.1, 1710 33.8 / 26.7; 256 x 256 stays for
 // 2560-5000 (46.2 / 54.9 at 3431) and from 5600 rows (101.5 / 120.5 at 9322).
+constexpr long long kCacheBytes = 256ll << 20;
 enum DenseTiles {
   kTiles32x64, kTiles64x64, kTiles64x128, kTiles96x128, kTiles128x128, kTiles128x256, kTiles256
 };
 static DenseTiles dense_tiling(int M, int N, int K, int cus, bool dense) {
-  if (dense && (long long)N * K * 2 > (256ll << 20) && M <= 256)
+  if (dense && (long long)N * K * 2 > kCacheBytes && M <= 256)
     return M <= 32 ? kTiles32x64 : M <= 64 ? kTiles64x128 : kTiles128x256;
   struct Kind {
     DenseTiles id;
@@ -1512,6 +1537,7 @@ static DenseTiles dense_tiling(int M, int N, int K, int cus, bool dense) {
 template <int MODE>
 static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int planes = 1) {
   p.col_major = nw > p.M;
+  p.rotate_k = (long long)nw * p.K * 2 > kCacheBytes;
 #define SYM_LAUNCH_SMALL(TM, TN, S, WM, WN)                                                      \
   hipLaunchKernelGGL((gemm_small_kernel<MODE, TM, TN, S, WM, WN>),                               \
                      dim3((nw + TN - 1) / TN, (p.M + TM - 1) / TM, planes), dim3(64 * WM * WN),  \
@@ -1838,6 +1864,7 @@ extern "C" int sym_moe_gate_up_fp8_tiled(const void* x, int T, int H, int I, int
   p.K = H;
   p.out_bf16 = (uint16_t*)h;
   p.tickets = (int*)workspace;
+  p.rotate_k = 1;
   (void)hipGetLastError();
   const int grid = std::max(8, sym_host::cu_count() / 8 * 8);
   hipLaunchKernelGGL((gemm_f8_persistent<kGateUp>), dim3(grid), dim3(f8::kThreads), 0,
@@ -1872,6 +1899,7 @@ extern "C" int sym_moe_down_fp8_tiled(const void* h, int T, int H, int I, int ro
   p.K = I;
   p.out_f32 = y;
   p.tickets = (int*)workspace;
+  p.rotate_k = 1;
   (void)hipGetLastError();
   const int grid = std::max(8, sym_host::cu_count() / 8 * 8);
   hipLaunchKernelGGL((gemm_f8_persistent<kDown>), dim3(grid), dim3(f8::kThreads), 0,
