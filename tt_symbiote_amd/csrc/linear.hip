@@ -534,6 +534,12 @@ static void launch_proj(const void* x, const void* w, const void* bias, int M, i
                        dim3(kLinThreads), 0, s, (const uint16_t*)x, (const uint16_t*)w,
                        (const uint16_t*)bias, M, N, K, (const uint16_t*)gamma, eps,
                        (const uint16_t*)residual, sumsq_parts, (uint16_t*)out_bf16, out_f32);
+  else if (M <= 16)
+    // one 16-row tile: half the activation loads in front of the norm (QKV at 7 rows 8.0 -> 7.4 us)
+    hipLaunchKernelGGL((proj_kernel<1, 4, NORM, RES>), dim3(N / 16), dim3(kLinThreads), 0, s,
+                       (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, M, N, K,
+                       (const uint16_t*)gamma, eps, (const uint16_t*)residual, sumsq_parts,
+                       (uint16_t*)out_bf16, out_f32);
   else
     hipLaunchKernelGGL((proj_kernel<2, 4, NORM, RES>), dim3(N / 16), dim3(kLinThreads), 0, s,
                        (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, M, N, K,
