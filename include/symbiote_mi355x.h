@@ -382,6 +382,9 @@ int sym_moe_down_fp8(const void* h, int T, int H, int I, const int32_t* seg_expe
  *   taken in fp32 in the epilogue: the dense projection plus the decoder layer's first residual
  *   add at sequence length > 1 (ttnn_attention.py:2211-2230 dense, modeling_bailing_moe_v2.py:
  *   457-460 residual). Same shape rules as sym_gemm_bf16; residual 8-byte aligned.
+ * sym_gemm_bf16_ws: sym_gemm_bf16 with a workspace of sym_gemm_splitk_workspace_bytes(M, N, K) bytes
+ *   (16-byte aligned; any contents). Where that is not 0 the product is split along K and its
+ *   fp32 partial sums go through the workspace (few output tiles, long K).
  * sym_gemm_swiglu_bf16: h[M, I] = silu(x . w[:I]^T) * (x . w[I:]^T) (bf16, w [2I, K]): the gate and
  *   up projections of a dense MLP (TTNNBailingMoeV2MLP) in one product. I % 64 == 0, K % 64 == 0;
  *   x, w and h 16-byte aligned; x and w each under 4 GB.
@@ -407,6 +410,10 @@ int sym_gemm_bf16(const void* a, const void* w, const void* bias, const float* r
                   int N, int K, void* out, int out_fp32, void* stream);
 int sym_gemm_bf16_res_bf16(const void* a, const void* w, const void* bias, const void* residual,
                            int M, int N, int K, float* out, void* stream);
+size_t sym_gemm_splitk_workspace_bytes(int M, int N, int K);
+int sym_gemm_bf16_ws(const void* a, const void* w, const void* bias, const float* residual, int M,
+                     int N, int K, void* out, int out_fp32, void* workspace,
+                     size_t workspace_bytes, void* stream);
 int sym_gemm_swiglu_bf16(const void* x, const void* w, int M, int I, int K, void* h, void* stream);
 int sym_moe_gate_up_tiled(const void* x, int T, int H, int I, int rows,
                           const int32_t* sorted_tokens, const int32_t* seg_expert,

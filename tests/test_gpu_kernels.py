@@ -491,6 +491,7 @@ def test_gemm_tiled(device, M, N, K, bias, res, out_dtype):
     (1000, 2064, 256), (900, 2048, 448),                  # 64 x 128
     (1500, 3072, 64), (2101, 2048, 5120),                 # 96 x 128
     (3431, 2048, 192), (5400, 3088, 128),                 # 128 x 128
+    (1, 2048, 5120), (70, 1040, 4160), (129, 1024, 4096), (250, 512, 8256),  # split along K
     (17, 131200, 1024), (50, 131216, 1024), (129, 131088, 1088),  # weights over 256 MB
 ])
 @pytest.mark.parametrize("kind", ["bf16", "f32", "bias_res32", "res16"])

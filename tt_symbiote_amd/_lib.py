@@ -129,6 +129,11 @@ _SIGNATURES = {
     ),
     "sym_gemm_bf16": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp, _c_int, _vp]),
     "sym_gemm_bf16_res_bf16": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp, _vp]),
+    "sym_gemm_splitk_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),
+    "sym_gemm_bf16_ws": (
+        _c_int,
+        [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp, _c_int, _vp, _c_size, _vp],
+    ),
     "sym_gemm_swiglu_bf16": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _vp, _vp]),
     "sym_moe_tiled_workspace_bytes": (_c_size, []),
     "sym_moe_gate_up_tiled": (

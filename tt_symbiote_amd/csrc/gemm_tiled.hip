@@ -74,6 +74,7 @@ struct TileArgs {
   int full_rt;              // DENSE with tail_rows > 0: row tiles 0 .. full_rt - 1 have TM rows,
   int tail_rows;            // the rows from full_rt * TM on tiles of tail_rows (one plane)
   int col_major;            // DENSE: the row tiles of a column tile are neighbours (N > M)
+  int split_steps;          // DENSE small tiles: grid z takes so many K-steps (0: all of K)
   int rotate_k;             // K-steps start at the column tile's index (KOrder)
   int* tickets;             // persistent grids: the caller's 8 per-XCD tile counters
   const float* w_scale;     // fp8 weights: [S, rows / 128, K / 128] block scales
@@ -1326,7 +1327,13 @@ __device__ __forceinline__ void small_tile(TileArgs p, const TileLoc& loc, uint1
   // rows do computes nothing (it still loads and syncs)
   const bool a_on = !kRagged || wave * (TM / kW) < loc.rows;
   const bool m_on = !kRagged || wm * kWR < loc.rows;
-  const int nk = p.K / kTK;
+  int nk = p.K / kTK;
+  if (p.split_steps > 0) {  // K-steps [z split_steps, ..) of the whole product, into plane z
+    const int s0 = loc.z * p.split_steps;
+    nk = min(p.split_steps, nk - s0);
+    p.a += s0 * kTK;
+    wbase += s0 * kTK;
+  }
   const KOrder kk_of = k_order(loc, nk, !kRagged && p.rotate_k);
   auto issue_a = [&](int kt) {
     if (!a_on) return;
@@ -1533,6 +1540,56 @@ static DenseTiles dense_tiling(int M, int N, int K, int cus, bool dense) {
   return id;
 }
 
+// Sum of the split-K planes, in plane order, plus bias and residual: 4 columns per thread.
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(
+    const float* __restrict__ parts, int splits, long long plane, int N,
+    const uint16_t* __restrict__ bias, const float* __restrict__ residual,
+    uint16_t* __restrict__ out_bf16, float* __restrict__ out_f32) {
+  const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (e >= plane) return;
+  const int col = (int)(e % N);
+  constexpr int kBatch = 8;  // planes in flight
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int z0 = 0; z0 < splits; z0 += kBatch) {
+    float4 t[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      t[i] = *reinterpret_cast<const float4*>(parts + min(z0 + i, splits - 1) * plane + e);
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      if (z0 + i < splits) {
+        v[0] += t[i].x; v[1] += t[i].y; v[2] += t[i].z; v[3] += t[i].w;
+      }
+  }
+  if (bias) {
+    const uint2 b = *reinterpret_cast<const uint2*>(bias + col);
+    v[0] += bf16_lo(b.x); v[1] += bf16_hi(b.x); v[2] += bf16_lo(b.y); v[3] += bf16_hi(b.y);
+  }
+  if (residual) {
+    const float4 r = *reinterpret_cast<const float4*>(residual + e);
+    v[0] += r.x; v[1] += r.y; v[2] += r.z; v[3] += r.w;
+  }
+  if (out_f32)
+    *reinterpret_cast<float4*>(out_f32 + e) = make_float4(v[0], v[1], v[2], v[3]);
+  else
+    *reinterpret_cast<uint2*>(out_bf16 + e) =
+        make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+}
+
+// K-splits of a dense product on 64 x 64 tiles, or 1: a long K over few tiles is a serial chain of
+// K-steps (about 0.3 us each) on an idle chip. Up to 8 splits of at least 8 steps, two
+// workgroups per CU, where the shorter chain is worth the partial sums and their launch: from 64
+// K-steps while the tiles fit the CUs, from 24 up to 64 rows. Measured (us in a replayed graph, one
+// chain against split): 2048 x 5120 at 1 row 22.7 / 8.1, 64 22.4 / 10.4, 128 22.4 / 14.2, 256 22.8
+// / 16.9, 500 28.8 / 24.1; 2048 x 2048 at 1 row 10.4 / 7.0, 64 10.4 / 8.5 (256: 10.8 / 13.1); the
+// shorter sums are also nearer to 64 bits (2048 x 5120, 64 rows: 3.7e-7 / 1.3e-7).
+static int dense_splits(int M, int N, int K, int cus) {
+  const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  const int steps = K / small::kTK;
+  if (tiles > cus || steps < (M <= 64 ? 24 : 64)) return 1;
+  return (int)std::min<long long>({2 * cus / tiles, steps / 8, 8});
+}
+
 // Small tiles of a dense product with nw weight rows (GATE_UP: 2 N).
 template <int MODE>
 static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int planes = 1) {
@@ -1557,7 +1614,8 @@ static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int p
 
 static int gemm_dense(const char* what, const void* a, const void* w, const void* bias,
                       const float* residual, const void* residual_bf16, int M, int N, int K,
-                      void* out, int out_fp32, void* stream) {
+                      void* out, int out_fp32, void* stream, void* workspace = nullptr,
+                      size_t workspace_bytes = 0) {
   SYM_REQUIRE(M >= 0, SYM_ERR_INVALID, "%s: M=%d < 0", what, M);
   if (M == 0) return SYM_OK;
   SYM_REQUIRE(a && w && out, SYM_ERR_INVALID, "%s: null pointer argument", what);
@@ -1588,6 +1646,28 @@ static int gemm_dense(const char* what, const void* a, const void* w, const void
   (void)hipGetLastError();
   const int cus = sym_host::cu_count();
   hipStream_t s = (hipStream_t)stream;
+  if (const int splits = workspace ? dense_splits(M, N, K, cus) : 1; splits > 1) {
+    const long long plane = (long long)M * N;
+    const size_t need = (size_t)splits * plane * sizeof(float);
+    SYM_REQUIRE(workspace_bytes >= need && aligned(workspace, 16), SYM_ERR_WORKSPACE,
+                "%s: workspace of %zu bytes (%zu needed, 16-byte aligned)", what, workspace_bytes,
+                need);
+    p.bias = nullptr;
+    p.residual = nullptr;
+    p.out_bf16 = nullptr;
+    p.out_f32 = (float*)workspace;
+    p.out_zstride = plane;
+    p.split_steps = (K / small::kTK + splits - 1) / splits;
+    // (whole splits only: the last one has at least one step)
+    const int planes = (K / small::kTK + p.split_steps - 1) / p.split_steps;
+    int rc = launch_small<kDense>(kTiles64x64, p, N, s, planes);
+    if (rc) return rc;
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((plane / 4 + 255) / 256)), dim3(256), 0,
+                       s, (const float*)workspace, planes, plane, N, (const uint16_t*)bias,
+                       residual, out_fp32 ? nullptr : (uint16_t*)out,
+                       out_fp32 ? (float*)out : nullptr);
+    return sym_host::check_launch("splitk_reduce_kernel");
+  }
   if (const DenseTiles id = dense_tiling(M, N, K, cus, true); id != kTiles256)
     return launch_small<kDense>(id, p, N, s);
   const int nx = (N + C::kTN - 1) / C::kTN;
@@ -1601,6 +1681,20 @@ static int gemm_dense(const char* what, const void* a, const void* w, const void
 extern "C" int sym_gemm_bf16(const void* a, const void* w, const void* bias, const float* residual,
                              int M, int N, int K, void* out, int out_fp32, void* stream) {
   return gemm_dense("gemm_bf16", a, w, bias, residual, nullptr, M, N, K, out, out_fp32, stream);
+}
+
+extern "C" size_t sym_gemm_splitk_workspace_bytes(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const int splits = dense_splits(M, N, K, sym_host::cu_count());
+  return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+}
+
+extern "C" int sym_gemm_bf16_ws(const void* a, const void* w, const void* bias,
+                                const float* residual, int M, int N, int K, void* out,
+                                int out_fp32, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+  return gemm_dense("gemm_bf16_ws", a, w, bias, residual, nullptr, M, N, K, out, out_fp32, stream,
+                    workspace, workspace_bytes);
 }
 
 extern "C" int sym_gemm_bf16_res_bf16(const void* a, const void* w, const void* bias,

@@ -177,10 +177,13 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
         _timed("gemm", lambda: _lib.call(
             "sym_gemm_bf16_res_bf16", _ptr(a), _ptr(w), _ptr(bias), _ptr(residual), M, N, K,
             _ptr(out), _stream()))
-    else:
-        _timed("gemm", lambda: _lib.call(
-            "sym_gemm_bf16", _ptr(a), _ptr(w), _ptr(bias), _ptr(residual), M, N, K, _ptr(out),
-            1 if out_dtype == torch.float32 else 0, _stream()))
+        return out
+    # long K over few output tiles: split along K, partial sums in a scratch tensor
+    ws_bytes = _lib.query("sym_gemm_splitk_workspace_bytes", M, N, K)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+    _timed("gemm", lambda: _lib.call(
+        "sym_gemm_bf16_ws", _ptr(a), _ptr(w), _ptr(bias), _ptr(residual), M, N, K, _ptr(out),
+        1 if out_dtype == torch.float32 else 0, _ptr(ws), ws_bytes, _stream()))
     return out
 
 

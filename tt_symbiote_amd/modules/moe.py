@@ -269,7 +269,7 @@ class HIPBailingMoeV2MLP(StatelessHIPModule):
         w_gate_up, w_down = self._dev["gate_up"], self._dev["down"]
         # two dense products, their tiles chosen from the row count (which the grouped kernels
         # know on the device only), the residual added in fp32 in the second one's epilogue: 64
-        # rows 191 -> 33 us, 2101 rows 207 -> 159 us at H = 2048, I = 5120. The grouped kernels
+        # rows 191 -> 23 us, 2101 rows 207 -> 159 us at H = 2048, I = 5120. The grouped kernels
         # keep the shapes these do not take as they did (H % 256, weights of 4 GB).
         if H % 256 == 0 and 2 * w_gate_up.numel() < 1 << 32:
             h = hip_ops.gemm_swiglu(x, w_gate_up[0])
