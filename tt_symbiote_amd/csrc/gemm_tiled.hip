@@ -1298,7 +1298,11 @@ constexpr int stage_elems(int tm, int tn) { return (tm + tn) * kTK; }
 
 // One TM x TN tile at loc. In grouped gate/up (kGather) the A rows wait for their token indices, so
 // the prologue's weight rows go first. hook() runs after the K loop, before the epilogue.
-template <int MODE, int TM, int TN, int S, int WM, int WN, bool kRagged, typename Hook>
+// kFold (fp32 outputs): the sums of each kFoldSteps K-steps are taken apart and then added up, 8
+// sums of 256 products each at K = 2048 instead of one of 2048: 1.0e-7 off 64 bits instead of
+// 2.7e-7 (the logits of an LM head).
+constexpr int kFoldSteps = 4;
+template <int MODE, int TM, int TN, int S, int WM, int WN, bool kRagged, bool kFold, typename Hook>
 __device__ __forceinline__ void small_tile(TileArgs p, const TileLoc& loc, uint16_t* smem,
                                            Hook hook) {
   using namespace small;
@@ -1359,6 +1363,18 @@ __device__ __forceinline__ void small_tile(TileArgs p, const TileLoc& loc, uint1
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  floatx4 tot[kFold ? NI : 1][kFold ? NJ : 1] = {};
+  auto fold = [&]() {
+    if constexpr (kFold) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          tot[i][j] += acc[i][j];
+          acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
 
   if constexpr (kGather) {
 #pragma unroll
@@ -1412,19 +1428,22 @@ __device__ __forceinline__ void small_tile(TileArgs p, const TileLoc& loc, uint1
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               __builtin_bit_cast(bf16x8, b[h][j]), __builtin_bit_cast(bf16x8, a[h][i]),
               acc[i][j], 0, 0, 0);
+    if (kFold && kt % kFoldSteps == kFoldSteps - 1) fold();
   }
+  fold();
   hook();
   const int col0 = MODE == kGateUp ? loc.ct * (TN / 2) + wn * (kWC / 2) : loc.ct * TN + wn * kWC;
-  store_block<MODE>(p, acc, loc, wm * kWR, col0, lane);
+  if constexpr (kFold) store_block<MODE>(p, tot, loc, wm * kWR, col0, lane);
+  else store_block<MODE>(p, acc, loc, wm * kWR, col0, lane);
 }
 
-template <int MODE, int TM, int TN, int S, int WM, int WN>
+template <int MODE, int TM, int TN, int S, int WM, int WN, bool kFold>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_small_kernel(TileArgs p) {
   __shared__ __align__(1024) uint16_t smem[S * small::stage_elems(TM, TN)];
   TileLoc loc;
   if (!locate_tile<kDense, TM>(p, threadIdx.x & 63, loc)) return;
-  small_tile<MODE, TM, TN, S, WM, WN, false>(p, loc, smem, NoHook{});
+  small_tile<MODE, TM, TN, S, WM, WN, false, kFold>(p, loc, smem, NoHook{});
 }
 
 // The grouped expert GEMMs on 64 x 128 tiles, two workgroups of 8 waves per CU, over the persistent
@@ -1442,7 +1461,7 @@ void gemm_narrow_persistent(TileArgs p, int nx) {
   __shared__ int s_next;
   static_assert(sizeof(smem) + sizeof(tab) + 16 <= 80 * 1024, "two workgroups per CU");
   walk_tiles<kNarrowTM, MODE>(p, nx, tab, s_next, [&](const TileLoc& loc, auto hook) {
-    small_tile<MODE, kNarrowTM, kNarrowTN, kNarrowS, 2, 4, true>(p, loc, smem, hook);
+    small_tile<MODE, kNarrowTM, kNarrowTN, kNarrowS, 2, 4, true, false>(p, loc, smem, hook);
   });
 }
 
@@ -1497,7 +1516,7 @@ static void dense_tail_split(int M, int nx, int cus, int& full_rt, int& tail_row
 // A weight too large for the caches (over kCacheBytes, e.g. an LM head) streams from HBM whatever the
 // tile, so the one with the fewest operand re-reads that covers M is taken (157184 x 2048, us,
 // 256 x 256 tiles against the choice): 32 rows 161 / 126 on 32 x 64; 64: 176 / 136 on 64 x 128;
-// 96: 189 / 149, 128: 198 / 168, 256: 272 / 209 on 128 x 256 (16: 154 / 119).
+// 96: 189 / 152, 128: 198 / 168, 256: 272 / 209 on 128 x 256 (16: 154 / 119).
 // Otherwise by estimated time: at K = 2048 a workgroup alone on its CU takes `alone` us and each
 // further one on the busiest CU `more`, with the load halfway between the mean and the busiest
 // CU's (fitted to sweeps of M = 16 .. 9322 at N = 2048 and 3072, K = 2048 and 5120; time scales
@@ -1591,12 +1610,12 @@ static int dense_splits(int M, int N, int K, int cus) {
 }
 
 // Small tiles of a dense product with nw weight rows (GATE_UP: 2 N).
-template <int MODE>
-static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int planes = 1) {
+template <int MODE, bool kFold>
+static int launch_small_as(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int planes) {
   p.col_major = nw > p.M;
   p.rotate_k = (long long)nw * p.K * 2 > kCacheBytes;
 #define SYM_LAUNCH_SMALL(TM, TN, S, WM, WN)                                                      \
-  hipLaunchKernelGGL((gemm_small_kernel<MODE, TM, TN, S, WM, WN>),                               \
+  hipLaunchKernelGGL((gemm_small_kernel<MODE, TM, TN, S, WM, WN, kFold>),                        \
                      dim3((nw + TN - 1) / TN, (p.M + TM - 1) / TM, planes), dim3(64 * WM * WN),  \
                      0, s, p);                                                                   \
   break
@@ -1610,6 +1629,13 @@ static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int p
   }
 #undef SYM_LAUNCH_SMALL
   return sym_host::check_launch("gemm_small_kernel");
+}
+template <int MODE>
+static int launch_small(DenseTiles id, TileArgs& p, int nw, hipStream_t s, int planes = 1) {
+  if constexpr (MODE == kDense) {
+    if (p.out_f32) return launch_small_as<MODE, true>(id, p, nw, s, planes);
+  }
+  return launch_small_as<MODE, false>(id, p, nw, s, planes);
 }
 
 static int gemm_dense(const char* what, const void* a, const void* w, const void* bias,
@@ -1775,7 +1801,7 @@ extern "C" int sym_moe_router_logits_split(const void* x, const void* w_planes, 
   (void)hipGetLastError();
   hipStream_t s = (hipStream_t)stream;
   // the tiles of one product with 3 E columns, one plane per grid z (E = 256, H = 2048, us,
-  // against 128 x 256 tiles of 32-column steps: 9322 tokens 48 / 35, 3431 41 / 24)
+  // against 128 x 256 tiles of 32-column steps: 9322 tokens 48 / 38, 3431 41 / 24)
   const DenseTiles id = dense_tiling(T, 3 * E, H, sym_host::cu_count(), false);
   if (id != kTiles256) return launch_small<kDense>(id, p, E, s, 3);
   hipLaunchKernelGGL((gemm_tile_kernel<kDense>),
