@@ -179,7 +179,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
             _ptr(out), _stream()))
         return out
     # long K over few output tiles: split along K, partial sums in a scratch tensor
-    ws_bytes = _lib.query("sym_gemm_splitk_workspace_bytes", M, N, K)
+    ws_bytes = (_lib.query("sym_gemm_splitk_workspace_bytes", M, N, K)
+                if K >= 4096 or (K >= 1536 and M <= 64) else 0)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
     _timed("gemm", lambda: _lib.call(
         "sym_gemm_bf16_ws", _ptr(a), _ptr(w), _ptr(bias), _ptr(residual), M, N, K, _ptr(out),
@@ -760,8 +761,10 @@ def moe_router_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return parts
 
 
-ROUTER_SPLIT_MIN_TOKENS = 1536  # from this many tokens the router logits run on bf16 MFMA tiles
-# (measured: 26 against 33 us at 1024 tokens, 48 against 34 us at 2048)
+# From this many tokens the router logits run on bf16 MFMA tiles (us, the fp32 kernel against them:
+# 333 tokens 11.3 / 11.1, 400 13.2 / 11.0, 640 16.3 / 11.5, 1024 24.2 / 13.5; 1.6e-7 against 1.1e-7
+# off 64 bits).
+ROUTER_SPLIT_MIN_TOKENS = 384
 
 
 def split_router_weight(w: torch.Tensor) -> torch.Tensor:

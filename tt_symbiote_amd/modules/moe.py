@@ -154,7 +154,9 @@ class HIPBailingMoE(StatelessHIPModule):
     def route(self, x: torch.Tensor) -> hip_ops.RouteResult:
         """Router logits (fp32 MFMA, or for many tokens bf16 MFMA tiles over the exact
         three-plane split of the fp32 gate weight) + fused top-k/permute for x [T, H] (bf16)."""
-        if x.shape[0] >= hip_ops.ROUTER_SPLIT_MIN_TOKENS:
+        T, H = x.shape
+        # (below 1536 tokens hidden sizes that the fp32 kernel does not take stay refused)
+        if T >= hip_ops.ROUTER_SPLIT_MIN_TOKENS and (H % 512 == 0 or T >= 1536):
             logits = hip_ops.moe_router_logits_split(x, self._dev["gate_w_planes"])
         else:
             logits = hip_ops.moe_router_logits(x, self._dev["gate_w"])
