@@ -329,6 +329,22 @@ int sym_moe_route_permute(const float* logits, int n_logit_parts, const float* b
                           int32_t* seg_offset, int32_t* seg_count, int32_t* n_segments,
                           void* workspace, size_t workspace_bytes, void* stream);
 
+/* The router alone (topk_idx, topk_w as sym_moe_route_permute gives them). */
+int sym_moe_route(const float* logits, int n_logit_parts, const float* bias, int T, int E,
+                  int n_group, int topk_group, int top_k, float routed_scale, int renormalize,
+                  int32_t* topk_idx, float* topk_w, void* stream);
+
+/* The MoE block of at most 4 tokens by token, without a permutation: experts
+ * topk_idx [T, top_k] and, with_shared, slot E of the stacks; out[t] = sum_k w y_k (+ shared)
+ * (+ residual[t], fp32), bf16 (TTNNExperts.forward, ttnn_moe.py:1159-1343, at decode). Weights
+ * bf16, or fp8 e4m3fn with the block scales s_gate_up and s_down (both null for bf16); h: scratch
+ * [T * top_k (+ T), I] bf16. I <= 512; shapes otherwise as sym_moe_grouped_swiglu. */
+int sym_moe_token_swiglu(const void* x, int T, int H, int I, const int32_t* topk_idx,
+                         const float* topk_w, int top_k, int E, int with_shared,
+                         const void* w_gate_up, const float* s_gate_up, const void* w_down,
+                         const float* s_down, const float* residual, void* h, void* out,
+                         void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * Grouped SwiGLU expert GEMMs over the segment list of sym_moe_route_permute.
  * Replaces the three sparse_matmul calls + silu/mul of TTNNExperts.forward

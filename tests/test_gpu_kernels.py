@@ -383,6 +383,35 @@ def test_grouped_swiglu(device, T, E, H, I, top_k, skew, kernel):
         assert torch.equal(yb.cpu(), yk.bfloat16())
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("T,E,H,I,top_k,shared,residual", [
+    (1, 256, 2048, 512, 8, True, True),
+    (4, 64, 512, 128, 4, True, False),
+    (3, 64, 1024, 384, 12, False, True),     # more assignments than waves
+    (2, 64, 512, 256, 32, True, True),       # the largest top_k; tokens that share experts
+])
+def test_moe_by_token(device, T, E, H, I, top_k, shared, residual, fp8):
+    """The MoE block by token gives the grouped path's bits (route, products and sums are the
+    same, in the same order)."""
+    g = torch.Generator(device=device).manual_seed(T + I)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=device)  # noqa: E731
+    moe = ts.HIPBailingMoE.from_weights(
+        gate_weight=rnd(E, H) * 0.02, expert_bias=rnd(E) * 0.01,
+        w_gate_up=(rnd(E, 2 * I, H) * 0.05).bfloat16(), w_down=(rnd(E, H, I) * 0.05).bfloat16(),
+        shared_gate_up=(rnd(2 * I, H) * 0.05).bfloat16() if shared else None,
+        shared_down=(rnd(H, I) * 0.05).bfloat16() if shared else None, top_k=top_k, n_group=8,
+        topk_group=4, routed_scaling_factor=2.5,
+        weight_format="fp8_e4m3" if fp8 else "bf16")
+    ts.set_device(moe, device)
+    x = rnd(T, H).bfloat16()
+    res = rnd(T, H) if residual else None
+    assert moe._by_token(T)
+    got = moe(x, residual=res)
+    moe.keep_last_route = True
+    assert not moe._by_token(T)
+    assert torch.equal(got, moe(x, residual=res))
+
+
 @pytest.mark.parametrize("T,E,H,I,top_k", [
     (40, 64, 256, 64, 6),      # below 12 rows per entry: thin tiles, one K-step down
     (700, 64, 256, 64, 6),     # above 60: whole 256 x 256 tiles, one K-step down

@@ -97,6 +97,16 @@ _SIGNATURES = {
         [_vp, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _vp,
          _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_size, _vp],
     ),
+    "sym_moe_route": (
+        _c_int,
+        [_vp, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _vp, _vp,
+         _vp],
+    ),
+    "sym_moe_token_swiglu": (
+        _c_int,
+        [_vp, _c_int, _c_int, _c_int, _vp, _vp, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp,
+         _vp, _vp, _vp],
+    ),
     "sym_moe_grouped_swiglu": (
         _c_int,
         [_vp, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _vp, _vp],

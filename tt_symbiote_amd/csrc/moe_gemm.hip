@@ -113,7 +113,8 @@ constexpr int kKLane = 16, kKHalf = 8;   // a lane's two loads are 32 contiguous
 // then the MFMAs, kept in that order by scheduling barriers. The 16 token indices of the pass
 // are read with scalar loads after the first weight batch is issued: waiting for them (lgkmcnt)
 // does not wait for the weights in flight (vmcnt).
-template <int U>
+// ONE: `rows` is the token of every lane (tok_rows is not read).
+template <int U, bool ONE = false>
 __device__ __forceinline__ void gate_up_pass(const uint16_t* __restrict__ x, int H,
                                              const int32_t* __restrict__ tok_rows, int rows,
                                              const uint16_t* __restrict__ wg,
@@ -123,7 +124,7 @@ __device__ __forceinline__ void gate_up_pass(const uint16_t* __restrict__ x, int
   accu = floatx4{0.f, 0.f, 0.f, 0.f};
   // the lane's token (rows past the pass read its last row, in bounds; their outputs are
   // dropped), loaded before the weights: waiting for it does not wait for them
-  const int tok = tok_rows[min(r16, rows - 1)];
+  const int tok = ONE ? rows : tok_rows[min(r16, rows - 1)];
   __builtin_amdgcn_sched_barrier(0);
   const uint16_t* xr = x + kq * kKLane;
   for (int st = s_beg; st < s_end; st += U) {
@@ -453,7 +454,7 @@ __device__ __forceinline__ uint4 ld16b(const uint8_t* p) {
 
 // gate/up over 16 rows of a segment, K-steps [s_beg, s_end) of 128 (a multiple of U); sg / su
 // point at the scales of this wave's gate / up row block, one per K-step.
-template <int U>
+template <int U, bool ONE = false>
 __device__ __forceinline__ void gate_up_pass_fp8(const uint16_t* __restrict__ x, int H,
                                                  const int32_t* __restrict__ tok_rows, int rows,
                                                  const uint8_t* __restrict__ wg,
@@ -465,7 +466,7 @@ __device__ __forceinline__ void gate_up_pass_fp8(const uint16_t* __restrict__ x,
   accg = floatx4{0.f, 0.f, 0.f, 0.f};
   accu = floatx4{0.f, 0.f, 0.f, 0.f};
   // the lane's token, loaded before the weights (see gate_up_pass)
-  const int tok = tok_rows[min(r16, rows - 1)];
+  const int tok = ONE ? rows : tok_rows[min(r16, rows - 1)];
   __builtin_amdgcn_sched_barrier(0);
   const uint16_t* xr = x + kq * 32;
   for (int st = s_beg; st < s_end; st += U) {
@@ -718,6 +719,124 @@ __global__ __launch_bounds__(kGemmThreads) void moe_down_fp8_lds_kernel(
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same products for a few tokens (kTokenMax), by token instead of by expert: at 1 to 4 tokens
+// hardly any expert is chosen twice, so sorting the assignments saves no weight traffic, and a
+// decode step at that size is a chain of launches. Assignment a = t K + k (shared expert: rows T K +
+// t) takes its expert straight from topk_idx, so no permute runs, and the down kernel owns all
+// assignments of a token's 16 columns, so it combines them itself (same order and rounding as
+// moe_combine_kernel): two launches fewer, the same bits. Measured
+// (us, the MoE block by expert against by token): bf16 1 token 32.9 / 29.0, 2 40.7 / 35.9, 4 54.5 /
+// 51.9, 5 61.8 / 63.6, 8 80.2 / 90.1; fp8 1 token 26.0 / 20.7, 4 38.7 / 35.2, 8 52.8 / 53.0.
+constexpr int kTokenMax = 4;
+
+struct TokItem {
+  int t, e;
+};
+__device__ __forceinline__ TokItem token_item(const int32_t* __restrict__ topk_idx, int a, int T,
+                                              int K, int E) {
+  const int tk = T * K;
+  return a < tk ? TokItem{a / K, __builtin_amdgcn_readfirstlane(topk_idx[a])} : TokItem{a - tk, E};
+}
+
+// grid: (I / 16 tiles) x (T K + T with the shared expert)
+template <int U, bool FP8>
+__global__ __launch_bounds__(kGemmThreads) void moe_gate_up_tok_kernel(
+    const uint16_t* __restrict__ x, int T, int K, int E, int H, int I,
+    const int32_t* __restrict__ topk_idx, const void* __restrict__ w_gu,
+    const float* __restrict__ s_gu, uint16_t* __restrict__ h) {
+  __shared__ float s_red[4][1][2][4][64];
+  const int a = blockIdx.y, col0 = blockIdx.x * 16;
+  const TokItem m = token_item(topk_idx, a, T, K, E);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int r16 = lane & 15, kq = lane >> 4;
+  floatx4 accg[1], accu[1];
+  if constexpr (FP8) {
+    const int nsteps = H >> 7;
+    const int s_beg = (wave * nsteps) >> 2, s_end = ((wave + 1) * nsteps) >> 2;
+    const uint8_t* wg = (const uint8_t*)w_gu + ((size_t)m.e * 2 * I + col0 + r16) * (size_t)H + kq * 32;
+    const float* sg = s_gu + ((size_t)m.e * ((2 * I) >> 7) + (col0 >> 7)) * nsteps;
+    const float* su = s_gu + ((size_t)m.e * ((2 * I) >> 7) + ((I + col0) >> 7)) * nsteps;
+    gate_up_pass_fp8<U, true>(x, H, nullptr, m.t, wg, wg + (size_t)I * H, sg, su, s_beg, s_end, r16, kq, accg[0],
+                        accu[0]);
+  } else {
+    const int nsteps = H >> 6;
+    const int s_beg = (wave * nsteps) >> 2, s_end = ((wave + 1) * nsteps) >> 2;
+    const uint16_t* wg =
+        (const uint16_t*)w_gu + ((size_t)m.e * 2 * I + col0 + r16) * (size_t)H + kq * kKLane;
+    gate_up_pass<U, true>(x, H, nullptr, m.t, wg, wg + (size_t)I * H, s_beg, s_end, r16, kq, accg[0], accu[0]);
+  }
+  gate_up_epilogue<1>(s_red, accg, accu, wave, lane, 1, (size_t)a, I, col0, h);
+}
+
+// grid: (H / 16) x T; a wave per assignment (kTokWaves at a time), all of I (NS K-steps) in
+// registers. Only row 0 of the MFMA tile is a row of h; the others repeat it.
+constexpr int kTokWaves = 9;
+constexpr int kTokItems = 33;  // top_k <= 32 assignments and the shared expert's
+template <int NS, bool FP8>
+__global__ __launch_bounds__(64 * kTokWaves) void moe_down_tok_kernel(
+    const uint16_t* __restrict__ h, int T, int K, int E, int with_shared, int H, int I,
+    const int32_t* __restrict__ topk_idx, const float* __restrict__ topk_w,
+    const void* __restrict__ w_d, const float* __restrict__ s_d,
+    const float* __restrict__ residual, uint16_t* __restrict__ out) {
+  __shared__ float s_y[kTokItems][16];
+  const int t = blockIdx.y, col0 = blockIdx.x * 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int items = K + (with_shared ? 1 : 0);
+  for (int i = wave; i < items; i += blockDim.x >> 6) {
+    const int a = i < K ? t * K + i : T * K + t;
+    const int e = token_item(topk_idx, a, T, K, E).e;
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (FP8) {
+      const uint8_t* wd = (const uint8_t*)w_d + ((size_t)e * H + col0 + r16) * (size_t)I + kq * 32;
+      const float* sd = s_d + ((size_t)e * (H >> 7) + (col0 >> 7)) * NS;
+      const uint16_t* hr = h + (size_t)a * I + kq * 32;
+      uint4 b[NS][2];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        b[s][0] = ld16b(wd + (s << 7));
+        b[s][1] = ld16b(wd + (s << 7) + 16);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        uint4 f[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f[j] = ld16(hr + (s << 7) + 8 * j);
+        acc = mfma_fp8_step(f, b[s], acc, sd[s]);
+      }
+    } else {
+      const uint16_t* wd =
+          (const uint16_t*)w_d + ((size_t)e * H + col0 + r16) * (size_t)I + kq * kKLane;
+      const uint16_t* hr = h + (size_t)a * I + kq * kKLane;
+      uint4 b[NS][2];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        b[s][0] = ld16(wd + (s << 6));
+        b[s][1] = ld16(wd + (s << 6) + kKHalf);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        acc = mfma16x16x32(ld16(hr + (s << 6)), b[s][0], acc);
+        acc = mfma16x16x32(ld16(hr + (s << 6) + kKHalf), b[s][1], acc);
+      }
+    }
+    if (kq == 0) s_y[i][r16] = acc[0];
+  }
+  __syncthreads();
+  const int c = threadIdx.x;
+  if (c >= 16) return;
+  float v = 0.f;
+  for (int k = 0; k < K; ++k) v += topk_w[t * K + k] * s_y[k][c];
+  if (with_shared) v += s_y[K][c];
+  if (residual) v += residual[(size_t)t * H + col0 + c];
+  out[(size_t)t * H + col0 + c] = f32_to_bf16(v);
 }
 
 // 8 consecutive values of a y row (fp32, or bf16 widened exactly)
@@ -1025,4 +1144,64 @@ extern "C" int sym_moe_down_fp8(const void* h, int T, int H, int I, const int32_
   SYM_LAUNCH_DOWN_FP8(1);
 #undef SYM_LAUNCH_DOWN_FP8
   return sym_host::check_launch("moe_down_fp8_kernel");
+}
+
+// s_gate_up / s_down: block scales of fp8 weights, or both null for bf16 weights
+extern "C" int sym_moe_token_swiglu(const void* x, int T, int H, int I, const int32_t* topk_idx,
+                                    const float* topk_w, int top_k, int E, int with_shared,
+                                    const void* w_gate_up, const float* s_gate_up,
+                                    const void* w_down, const float* s_down,
+                                    const float* residual, void* h, void* out, void* stream) {
+  const bool fp8 = s_gate_up != nullptr;
+  int rc = fp8 ? check_fp8_gemm_args("moe_token_swiglu", T, H, I, 1)
+               : check_gemm_args("moe_token_swiglu", T, H, I, 1);
+  if (rc) return rc;
+  if (T == 0) return SYM_OK;
+  SYM_REQUIRE(x && topk_idx && topk_w && w_gate_up && w_down && h && out, SYM_ERR_INVALID,
+              "moe_token_swiglu: null pointer argument");
+  SYM_REQUIRE((s_gate_up == nullptr) == (s_down == nullptr), SYM_ERR_INVALID,
+              "moe_token_swiglu: scales for one weight only");
+  SYM_REQUIRE(T <= kTokenMax && I <= 512, SYM_ERR_UNSUPPORTED,
+              "moe_token_swiglu: T=%d above %d or I=%d above 512", T, kTokenMax, I);
+  SYM_REQUIRE(top_k >= 1 && top_k < kTokItems && E >= 1, SYM_ERR_INVALID,
+              "moe_token_swiglu: top_k=%d E=%d", top_k, E);
+  (void)hipGetLastError();
+  hipStream_t s = (hipStream_t)stream;
+  const dim3 g1(I / 16, T * (top_k + (with_shared ? 1 : 0))), b1(kGemmThreads);
+#define SYM_LAUNCH_GU_TOK(UU, F)                                                                  \
+  hipLaunchKernelGGL((moe_gate_up_tok_kernel<UU, F>), g1, b1, 0, s, (const uint16_t*)x, T, top_k, \
+                     E, H, I, topk_idx, w_gate_up, s_gate_up, (uint16_t*)h)
+  if (fp8) {
+    if ((H / 512) % 2 == 0) SYM_LAUNCH_GU_TOK(2, true);
+    else SYM_LAUNCH_GU_TOK(1, true);
+  } else {
+    const int wave_steps = H / 256;
+    if (wave_steps % 4 == 0) SYM_LAUNCH_GU_TOK(4, false);
+    else if (wave_steps % 2 == 0) SYM_LAUNCH_GU_TOK(2, false);
+    else SYM_LAUNCH_GU_TOK(1, false);
+  }
+#undef SYM_LAUNCH_GU_TOK
+  rc = sym_host::check_launch("moe_gate_up_tok_kernel");
+  if (rc) return rc;
+  const dim3 g2(H / 16, T), b2(64 * std::min(top_k + (with_shared ? 1 : 0), kTokWaves));
+#define SYM_LAUNCH_DN_TOK(NS, F)                                                                  \
+  case NS:                                                                                        \
+    hipLaunchKernelGGL((moe_down_tok_kernel<NS, F>), g2, b2, 0, s, (const uint16_t*)h, T, top_k, E, \
+                       with_shared, H, I, topk_idx, topk_w, w_down, s_down, residual,             \
+                       (uint16_t*)out);                                                           \
+    break;
+  if (fp8) {
+    switch (I / 128) {
+      SYM_LAUNCH_DN_TOK(1, true) SYM_LAUNCH_DN_TOK(2, true) SYM_LAUNCH_DN_TOK(3, true)
+      SYM_LAUNCH_DN_TOK(4, true)
+    }
+  } else {
+    switch (I / 64) {
+      SYM_LAUNCH_DN_TOK(1, false) SYM_LAUNCH_DN_TOK(2, false) SYM_LAUNCH_DN_TOK(3, false)
+      SYM_LAUNCH_DN_TOK(4, false) SYM_LAUNCH_DN_TOK(5, false) SYM_LAUNCH_DN_TOK(6, false)
+      SYM_LAUNCH_DN_TOK(7, false) SYM_LAUNCH_DN_TOK(8, false)
+    }
+  }
+#undef SYM_LAUNCH_DN_TOK
+  return sym_host::check_launch("moe_down_tok_kernel");
 }

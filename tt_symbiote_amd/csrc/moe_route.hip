@@ -771,6 +771,49 @@ extern "C" int sym_moe_router_logits_norm(const float* h, const float* ss_parts,
   return sym_host::check_launch("moe_router_logits_kernel");
 }
 
+static int check_route(const char* what, int n_logit_parts, int T, int E, int n_group,
+                       int topk_group, int top_k) {
+  SYM_REQUIRE(n_logit_parts >= 1 && n_logit_parts <= kLogitParts, SYM_ERR_INVALID,
+              "%s: n_logit_parts=%d out of [1,%d]", what, n_logit_parts, kLogitParts);
+  SYM_REQUIRE(E == 64 || E == 128 || E == 256 || E == 512, SYM_ERR_UNSUPPORTED,
+              "%s: E=%d not in {64,128,256,512}", what, E);
+  SYM_REQUIRE(n_group >= 1 && E % n_group == 0, SYM_ERR_INVALID,
+              "%s: n_group=%d does not divide E=%d", what, n_group, E);
+  const int epl = E / 64;
+  const int gsz = E / n_group;
+  SYM_REQUIRE(gsz >= 2 && gsz % epl == 0, SYM_ERR_UNSUPPORTED,
+              "%s: group size %d must be >= 2 and a multiple of %d", what, gsz, epl);
+  const int lpg = gsz / epl;
+  SYM_REQUIRE((lpg & (lpg - 1)) == 0, SYM_ERR_UNSUPPORTED,
+              "%s: lanes per group %d is not a power of two", what, lpg);
+  SYM_REQUIRE(top_k >= 1 && top_k <= kMaxTopK && top_k <= E, SYM_ERR_INVALID,
+              "%s: top_k=%d out of range", what, top_k);
+  SYM_REQUIRE(topk_group >= 1 && topk_group <= n_group, SYM_ERR_INVALID,
+              "%s: topk_group=%d out of range [1,%d]", what, topk_group, n_group);
+  SYM_REQUIRE(top_k <= topk_group * gsz, SYM_ERR_INVALID,
+              "%s: top_k=%d exceeds the experts of the kept groups", what, top_k);
+  SYM_REQUIRE((long long)T * top_k + T < (1ll << 30), SYM_ERR_INVALID,
+              "%s: T=%d too large", what, T);
+  return SYM_OK;
+}
+
+static int launch_route(const float* logits, int n_logit_parts, const float* bias, int T, int E,
+                        int n_group, int topk_group, int top_k, float routed_scale,
+                        int renormalize, int32_t* topk_idx, float* topk_w, hipStream_t s) {
+  const dim3 grid((T + 3) / 4), block(256);
+#define SYM_LAUNCH_ROUTE(EE)                                                                    \
+  hipLaunchKernelGGL(moe_route_kernel<EE>, grid, block, 0, s, logits, n_logit_parts, bias, T, E, \
+                     n_group, topk_group, top_k, routed_scale, renormalize, topk_idx, topk_w)
+  switch (E / 64) {
+    case 1: SYM_LAUNCH_ROUTE(1); break;
+    case 2: SYM_LAUNCH_ROUTE(2); break;
+    case 4: SYM_LAUNCH_ROUTE(4); break;
+    default: SYM_LAUNCH_ROUTE(8); break;
+  }
+#undef SYM_LAUNCH_ROUTE
+  return sym_host::check_launch("moe_route_kernel");
+}
+
 extern "C" int sym_moe_route_permute(const float* logits, int n_logit_parts, const float* bias,
                                      int T, int E, int n_group, int topk_group, int top_k,
                                      float routed_scale, int renormalize, int with_shared,
@@ -785,27 +828,8 @@ extern "C" int sym_moe_route_permute(const float* logits, int n_logit_parts, con
                   sorted_tokens && inv_perm && seg_expert && seg_offset && seg_count &&
                   n_segments,
               SYM_ERR_INVALID, "moe_route_permute: null pointer argument");
-  SYM_REQUIRE(n_logit_parts >= 1 && n_logit_parts <= kLogitParts, SYM_ERR_INVALID,
-              "moe_route_permute: n_logit_parts=%d out of [1,%d]", n_logit_parts, kLogitParts);
-  SYM_REQUIRE(E == 64 || E == 128 || E == 256 || E == 512, SYM_ERR_UNSUPPORTED,
-              "moe_route_permute: E=%d not in {64,128,256,512}", E);
-  SYM_REQUIRE(n_group >= 1 && E % n_group == 0, SYM_ERR_INVALID,
-              "moe_route_permute: n_group=%d does not divide E=%d", n_group, E);
-  const int epl = E / 64;
-  const int gsz = E / n_group;
-  SYM_REQUIRE(gsz >= 2 && gsz % epl == 0, SYM_ERR_UNSUPPORTED,
-              "moe_route_permute: group size %d must be >= 2 and a multiple of %d", gsz, epl);
-  const int lpg = gsz / epl;
-  SYM_REQUIRE((lpg & (lpg - 1)) == 0, SYM_ERR_UNSUPPORTED,
-              "moe_route_permute: lanes per group %d is not a power of two", lpg);
-  SYM_REQUIRE(top_k >= 1 && top_k <= kMaxTopK && top_k <= E, SYM_ERR_INVALID,
-              "moe_route_permute: top_k=%d out of range", top_k);
-  SYM_REQUIRE(topk_group >= 1 && topk_group <= n_group, SYM_ERR_INVALID,
-              "moe_route_permute: topk_group=%d out of range [1,%d]", topk_group, n_group);
-  SYM_REQUIRE(top_k <= topk_group * gsz, SYM_ERR_INVALID,
-              "moe_route_permute: top_k=%d exceeds the experts of the kept groups", top_k);
-  SYM_REQUIRE((long long)T * top_k + T < (1ll << 30), SYM_ERR_INVALID,
-              "moe_route_permute: T=%d too large", T);
+  int rc = check_route("moe_route_permute", n_logit_parts, T, E, n_group, topk_group, top_k);
+  if (rc) return rc;
   const size_t ws_need = sym_moe_route_workspace_bytes(T, E);
   SYM_REQUIRE(ws_need == 0 || (workspace && workspace_bytes >= ws_need), SYM_ERR_WORKSPACE,
               "moe_route_permute: workspace of %zu bytes needed for T=%d (got %zu)", ws_need, T,
@@ -813,6 +837,7 @@ extern "C" int sym_moe_route_permute(const float* logits, int n_logit_parts, con
 
   hipStream_t s = (hipStream_t)stream;
   (void)hipGetLastError();
+  const int epl = E / 64;
   if (T <= kFusedTokens) {
 #define SYM_LAUNCH_ROUTE_PERMUTE(EE)                                                             \
   hipLaunchKernelGGL(moe_route_permute_kernel<EE>, dim3(1), dim3(kPermuteThreads), 0, s, logits,  \
@@ -828,18 +853,8 @@ extern "C" int sym_moe_route_permute(const float* logits, int n_logit_parts, con
 #undef SYM_LAUNCH_ROUTE_PERMUTE
     return sym_host::check_launch("moe_route_permute_kernel");
   }
-  const dim3 grid((T + 3) / 4), block(256);
-#define SYM_LAUNCH_ROUTE(EE)                                                                    \
-  hipLaunchKernelGGL(moe_route_kernel<EE>, grid, block, 0, s, logits, n_logit_parts, bias, T, E, \
-                     n_group, topk_group, top_k, routed_scale, renormalize, topk_idx, topk_w)
-  switch (epl) {
-    case 1: SYM_LAUNCH_ROUTE(1); break;
-    case 2: SYM_LAUNCH_ROUTE(2); break;
-    case 4: SYM_LAUNCH_ROUTE(4); break;
-    default: SYM_LAUNCH_ROUTE(8); break;
-  }
-#undef SYM_LAUNCH_ROUTE
-  int rc = sym_host::check_launch("moe_route_kernel");
+  rc = launch_route(logits, n_logit_parts, bias, T, E, n_group, topk_group, top_k, routed_scale,
+                    renormalize, topk_idx, topk_w, s);
   if (rc) return rc;
   if (ws_need == 0) {
     hipLaunchKernelGGL(moe_permute_kernel, dim3(1), dim3(kPermuteThreads), 0, s, topk_idx, T,
@@ -861,4 +876,18 @@ extern "C" int sym_moe_route_permute(const float* logits, int n_logit_parts, con
   hipLaunchKernelGGL(moe_permute_scatter_kernel, dim3(n_chunks), dim3(256), 0, s, topk_idx, T,
                      top_k, E, chunk_cnt, expert_offsets, sorted_tokens, inv_perm);
   return sym_host::check_launch("moe_permute_scatter_kernel");
+}
+
+extern "C" int sym_moe_route(const float* logits, int n_logit_parts, const float* bias, int T, int E,
+                             int n_group, int topk_group, int top_k, float routed_scale,
+                             int renormalize, int32_t* topk_idx, float* topk_w, void* stream) {
+  SYM_REQUIRE(T >= 0, SYM_ERR_INVALID, "moe_route: T=%d < 0", T);
+  if (T == 0) return SYM_OK;
+  SYM_REQUIRE(logits && bias && topk_idx && topk_w, SYM_ERR_INVALID,
+              "moe_route: null pointer argument");
+  int rc = check_route("moe_route", n_logit_parts, T, E, n_group, topk_group, top_k);
+  if (rc) return rc;
+  (void)hipGetLastError();
+  return launch_route(logits, n_logit_parts, bias, T, E, n_group, topk_group, top_k, routed_scale,
+                      renormalize, topk_idx, topk_w, (hipStream_t)stream);
 }

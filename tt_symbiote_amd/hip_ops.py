@@ -1056,6 +1056,76 @@ def moe_grouped_swiglu(x: torch.Tensor, route: RouteResult, w_gate_up,
     return h, y
 
 
+# Up to this many tokens the MoE block runs by token (:func:`moe_token_swiglu`).
+MOE_TOKEN_MAX = 4
+
+
+def moe_route(logits: torch.Tensor, bias: torch.Tensor, *, n_group: int, topk_group: int,
+              top_k: int, routed_scale: float, renormalize: bool = True):
+    """The router alone, as in :func:`moe_route_permute`: (topk_idx [T, K] int32, topk_w [T, K])."""
+    _check(logits, "logits", torch.float32)
+    if logits.dim() != 3:
+        raise ValueError(f"logits must be [P, T, E], got {tuple(logits.shape)}")
+    n_parts, T, E = logits.shape
+    _check(bias, "bias", torch.float32, logits.device)
+    _check_shape(bias, "bias", (E,))
+    topk_idx = torch.empty(T, top_k, dtype=torch.int32, device=logits.device)
+    topk_w = torch.empty(T, top_k, dtype=torch.float32, device=logits.device)
+    _timed("moe_route_permute", lambda: _lib.call(
+        "sym_moe_route", _ptr(logits), n_parts, _ptr(bias), T, E, int(n_group), int(topk_group),
+        int(top_k), float(routed_scale), 1 if renormalize else 0, _ptr(topk_idx), _ptr(topk_w),
+        _stream()))
+    return topk_idx, topk_w
+
+
+def moe_token_swiglu(x: torch.Tensor, topk_idx: torch.Tensor, topk_w: torch.Tensor, w_gate_up,
+                     w_down, num_experts: int, with_shared: bool,
+                     residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The routed experts, the shared expert (slot ``num_experts`` of the stacks) and the weighted
+    sum of a few tokens x [T, H] (T <= MOE_TOKEN_MAX), straight from the router's choices:
+    bf16 [T, H], with ``residual`` (fp32) added before the rounding. Weights as in
+    :func:`moe_grouped_swiglu`; I <= 512."""
+    _check(x, "x", torch.bfloat16)
+    if x.dim() != 2:
+        raise ValueError(f"x must be [T, H], got {tuple(x.shape)}")
+    T, H = x.shape
+    dev = x.device
+    fp8 = isinstance(w_gate_up, BlockFp8)
+    if fp8 != isinstance(w_down, BlockFp8):
+        raise ValueError("w_gate_up and w_down must both be bf16 or both BlockFp8")
+    s_gate_up = s_down = None
+    if fp8:
+        w_gate_up.check("w_gate_up", dev)
+        w_down.check("w_down", dev)
+        s_gate_up, s_down = w_gate_up.scale, w_down.scale
+        w_gate_up, w_down = w_gate_up.q, w_down.q
+    else:
+        _check(w_gate_up, "w_gate_up", torch.bfloat16, dev)
+        _check(w_down, "w_down", torch.bfloat16, dev)
+    if w_gate_up.dim() != 3 or w_gate_up.shape[2] != H or w_gate_up.shape[1] % 2:
+        raise ValueError(f"w_gate_up must be [S, 2I, {H}], got {tuple(w_gate_up.shape)}")
+    S, I = w_gate_up.shape[0], w_gate_up.shape[1] // 2
+    _check_shape(w_down, "w_down", (S, H, I))
+    if S < num_experts + (1 if with_shared else 0):
+        raise ValueError(f"weight stack has {S} slots; {num_experts} experts"
+                         f"{' + shared' if with_shared else ''} needed")
+    _check(topk_idx, "topk_idx", torch.int32, dev)
+    K = topk_idx.shape[1] if topk_idx.dim() == 2 else 0
+    _check_shape(topk_idx, "topk_idx", (T, K))
+    _check(topk_w, "topk_w", torch.float32, dev)
+    _check_shape(topk_w, "topk_w", (T, K))
+    if residual is not None:
+        _check(residual, "residual", torch.float32, dev)
+        _check_shape(residual, "residual", (T, H))
+    h = torch.empty(T * K + (T if with_shared else 0), I, dtype=torch.bfloat16, device=dev)
+    out = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
+    _timed("moe_token_swiglu", lambda: _lib.call(
+        "sym_moe_token_swiglu", _ptr(x), T, H, I, _ptr(topk_idx), _ptr(topk_w), K,
+        int(num_experts), 1 if with_shared else 0, _ptr(w_gate_up), _ptr(s_gate_up),
+        _ptr(w_down), _ptr(s_down), _ptr(residual), _ptr(h), _ptr(out), _stream()))
+    return out
+
+
 def moe_unpermute_combine(y: torch.Tensor, route: RouteResult,
                           residual: Optional[torch.Tensor] = None,
                           out: Optional[torch.Tensor] = None) -> torch.Tensor:

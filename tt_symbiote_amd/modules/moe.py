@@ -165,6 +165,21 @@ class HIPBailingMoE(StatelessHIPModule):
             top_k=self.top_k, routed_scale=self.routed_scaling_factor, renormalize=True,
             with_shared=self.has_shared)
 
+    def _by_token(self, T: int) -> bool:
+        """Whether a batch of T tokens runs by token (sizes the token kernels take; a caller that
+        wants the permutation of ``last_route`` keeps the grouped path)."""
+        H, I = self.hidden_size, self.intermediate_size
+        whole = 128 if self.weight_format == "fp8_e4m3" else 64
+        return (0 < T <= hip_ops.MOE_TOKEN_MAX and not self.keep_last_route and I <= 512
+                and I % whole == 0 and H % (4 * whole) == 0)
+
+    def _tokens(self, x: torch.Tensor, logits: torch.Tensor, residual) -> torch.Tensor:
+        idx, w = hip_ops.moe_route(
+            logits, self._dev["bias"], n_group=self.n_group, topk_group=self.topk_group,
+            top_k=self.top_k, routed_scale=self.routed_scaling_factor, renormalize=True)
+        return hip_ops.moe_token_swiglu(x, idx, w, self._dev["gate_up"], self._dev["down"],
+                                        self.num_experts, self.has_shared, residual=residual)
+
     def forward(self, hidden_states: torch.Tensor, residual: torch.Tensor = None) -> torch.Tensor:
         """MoE output (bf16); with ``residual`` the result is residual + MoE(x) (one rounding)."""
         shape = hidden_states.shape
@@ -176,6 +191,9 @@ class HIPBailingMoE(StatelessHIPModule):
         res = None
         if residual is not None:
             res = residual.reshape(-1, H).to(torch.float32).contiguous()
+        if self._by_token(x.shape[0]):
+            logits = hip_ops.moe_router_logits(x, self._dev["gate_w"])
+            return self._tokens(x, logits, res).view(shape)
         route = self.route(x)
         if self.keep_last_route:
             self.last_route = route
@@ -192,6 +210,8 @@ class HIPBailingMoE(StatelessHIPModule):
         inside the router-logits kernel, which also hands the normalised rows to the experts."""
         parts, xn = hip_ops.moe_router_logits_norm(h, ss_parts, norm_weight, norm_eps,
                                                    self._dev["gate_w"])
+        if self._by_token(xn.shape[0]):
+            return self._tokens(xn, parts, h)
         route = hip_ops.moe_route_permute(
             parts, self._dev["bias"], n_group=self.n_group, topk_group=self.topk_group,
             top_k=self.top_k, routed_scale=self.routed_scaling_factor, renormalize=True,
