@@ -242,11 +242,13 @@ class HIPLMHead(StatelessHIPModule):
         shape = x.shape
         x2 = x.reshape(-1, self.hidden_size).to(torch.bfloat16).contiguous()
         V = self.vocab_size
-        # the tiled GEMM at every batch: its small tiles read the weight once for all rows, the
-        # decode projection once per 32 (V = 157184, H = 2048: 16 rows 119 against 150 us, 32 126
-        # against 288, 64 135 against 414; 1 row 109 against 114). It takes weights under 4 GB.
-        fits = 2 * max(V, x2.shape[0]) * self.hidden_size < 1 << 32
-        op = hip_ops.gemm if fits or x2.shape[0] > 64 else hip_ops.linear
+        # the tiled GEMM reads the weight once for all rows, the decode projection once per 32
+        # (16 without the norm): V = 157184, H = 2048, us, projection against GEMM: 2 rows 108.8 /
+        # 114.4, 4 110.4 / 115.6, 6 115.5 / 114.1, 16 147 / 120, 32 287 / 128, 64 414 / 136. The
+        # GEMM takes weights under 4 GB.
+        rows = x2.shape[0]
+        fits = 2 * max(V, rows) * self.hidden_size < 1 << 32
+        op = hip_ops.gemm if rows > 64 or (rows > 4 and fits) else hip_ops.linear
         tail = V % 16
         parts = []
         if V - tail:
