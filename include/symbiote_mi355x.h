@@ -233,6 +233,15 @@ int sym_attn_decode_step(const void* qkv, const void* q_norm_w, const void* k_no
  *   same workspace. The step appends the new token's k and v by the rule above before the
  *   attention reads the pool.
  */
+/* sym_paged_kv_fill_fp8_packed: the same for k, v [T, Hkv, head_dim] of packed sequences that start
+ *   at positions[cu[s]] of page-table row seq_ids[cu[s]] (positions, seq_ids [T]). */
+int sym_paged_kv_fill_fp8_packed(const void* k, const void* v, const int32_t* cu_seqlens,
+                                 const int32_t* positions, const int32_t* seq_ids, int T,
+                                 int n_seqs, int max_seqlen, int Hkv, int head_dim, void* k_pool,
+                                 void* v_pool, float* k_scale, float* v_scale,
+                                 const int32_t* block_tables, int page_table_rows,
+                                 int max_blocks_per_seq, int block_size, int num_blocks,
+                                 void* stream);
 int sym_paged_kv_fill_fp8(const void* k, const void* v, long long tok_stride,
                           long long head_stride, const int32_t* cu_seqlens,
                           const int32_t* start_pos, const int32_t* seq_rows, int n_seqs,

@@ -196,6 +196,36 @@ def test_kv_fill_fp8_bit_exact(device):
     assert np.array_equal(hip_ops.fp8_v_rows(vp.view(torch.uint8)).cpu().numpy(), ovp)
 
 
+def test_kv_fill_fp8_packed(device):
+    """Per-token starts and rows (with an empty sequence, also last) give the bytes of the
+    per-sequence ones."""
+    lens, starts, rows, Hkv, bs = [5, 0, 40, 17, 0], [3, 0, 30, 0, 0], [2, 0, 1, 3, 0], 2, 16
+    g = torch.Generator(device=device).manual_seed(5)
+    T = sum(lens)
+    k, v = (torch.randn(T, Hkv, 128, generator=g, device=device).bfloat16() for _ in range(2))
+    i32 = dict(dtype=torch.int32, device=device)
+    cu = torch.tensor([0] + lens, **i32).cumsum(0).int()
+    pt = torch.randperm(20, generator=g, device=device)[:20].int().view(4, 5).contiguous()
+    seq = [s for s, n in enumerate(lens) for _ in range(n)]
+    pos = torch.tensor([starts[s] + i for s, n in enumerate(lens) for i in range(n)], **i32)
+    got = []
+    for packed in (False, True):
+        pools = [torch.zeros(20, Hkv, bs, 128, device=device).to(torch.float8_e4m3fn),
+                 torch.zeros(20, Hkv, 128, bs, device=device).to(torch.float8_e4m3fn),
+                 torch.zeros(20, Hkv, device=device), torch.zeros(20, Hkv, device=device)]
+        if packed:
+            hip_ops.paged_kv_fill_fp8_packed(k, v, cu, 40, pos,
+                                             torch.tensor([rows[s] for s in seq], **i32), *pools,
+                                             pt)
+        else:
+            hip_ops.paged_kv_fill_fp8(k, v, cu, 40, *pools, pt,
+                                      start_pos=torch.tensor(starts, **i32),
+                                      seq_rows=torch.tensor(rows, **i32))
+        got.append([p.view(torch.uint8) if p.dtype == torch.float8_e4m3fn else p for p in pools])
+    assert float(got[0][2].max()) > 0
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 def test_kv_fill_fp8_htd_layout_and_skips(device):
     """[Hkv, S, D] input (paged_fill_on_device's layout) equals the [S, Hkv, D] one; a negative
     start skips the sequence."""

@@ -879,16 +879,18 @@ __device__ __forceinline__ uint2 byte_mask8(uint32_t m) {
 __global__ __launch_bounds__(256) void paged_kv_fill_fp8_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, long long tok_stride,
     long long head_stride, const int32_t* __restrict__ cu_seqlens,
-    const int32_t* __restrict__ start_pos, const int32_t* __restrict__ seq_rows, int n_rows,
-    int Hkv, uint8_t* __restrict__ k_pool, uint8_t* __restrict__ v_pool,
+    const int32_t* __restrict__ start_pos, const int32_t* __restrict__ seq_rows, int n_tok,
+    int n_rows, int Hkv, uint8_t* __restrict__ k_pool, uint8_t* __restrict__ v_pool,
     float* __restrict__ k_scale, float* __restrict__ v_scale,
     const int32_t* __restrict__ block_tables, int mbps, int block_size, int num_blocks) {
   __shared__ float s_amax[2][4];
   const int j = blockIdx.x, g = blockIdx.y, sq = blockIdx.z;
   const int c0 = cu_seqlens[sq];
   const int L = cu_seqlens[sq + 1] - c0;
-  const int start = start_pos ? start_pos[sq] : 0;
-  const int row = seq_rows ? seq_rows[sq] : sq;  // page-table row of the sequence
+  // n_tok > 0: start_pos and seq_rows are per token, a sequence's are its first token's
+  const int si = n_tok > 0 ? min(max(c0, 0), n_tok - 1) : sq;
+  const int start = start_pos ? start_pos[si] : 0;
+  const int row = seq_rows ? seq_rows[si] : sq;  // page-table row of the sequence
   if (L <= 0 || start < 0 || row < 0 || row >= n_rows) return;
   const int blk = start / block_size + j;
   const int p0 = max(start, blk * block_size);
@@ -1726,14 +1728,14 @@ extern "C" int sym_attn_decode_step_fp8(const void* qkv, const void* q_norm_w,
                        workspace_bytes, out, stream);
 }
 
-extern "C" int sym_paged_kv_fill_fp8(const void* k, const void* v, long long tok_stride,
-                                     long long head_stride, const int32_t* cu_seqlens,
-                                     const int32_t* start_pos, const int32_t* seq_rows,
-                                     int n_seqs, int max_seqlen, int Hkv, int head_dim,
-                                     void* k_pool, void* v_pool, float* k_scale, float* v_scale,
-                                     const int32_t* block_tables, int page_table_rows,
-                                     int max_blocks_per_seq, int block_size, int num_blocks,
-                                     void* stream) {
+static int kv_fill_fp8(const void* k, const void* v, long long tok_stride,
+                      long long head_stride, const int32_t* cu_seqlens,
+                      const int32_t* start_pos, const int32_t* seq_rows, int n_tok,
+                      int n_seqs, int max_seqlen, int Hkv, int head_dim,
+                      void* k_pool, void* v_pool, float* k_scale, float* v_scale,
+                      const int32_t* block_tables, int page_table_rows,
+                      int max_blocks_per_seq, int block_size, int num_blocks,
+                      void* stream) {
   int rc = check_cache_args("paged_kv_fill_fp8", n_seqs, Hkv, head_dim, block_size,
                             max_blocks_per_seq, num_blocks);
   if (rc) return rc;
@@ -1755,8 +1757,37 @@ extern "C" int sym_paged_kv_fill_fp8(const void* k, const void* v, long long tok
   (void)hipGetLastError();
   hipLaunchKernelGGL(paged_kv_fill_fp8_kernel, dim3(gx, Hkv, n_seqs), dim3(256), 0,
                      (hipStream_t)stream, (const uint16_t*)k, (const uint16_t*)v, tok_stride,
-                     head_stride, cu_seqlens, start_pos, seq_rows, page_table_rows, Hkv,
+                     head_stride, cu_seqlens, start_pos, seq_rows, n_tok, page_table_rows,
+                     Hkv,
                      (uint8_t*)k_pool, (uint8_t*)v_pool, k_scale, v_scale, block_tables,
                      max_blocks_per_seq, block_size, num_blocks);
   return sym_host::check_launch("paged_kv_fill_fp8_kernel");
+}
+
+extern "C" int sym_paged_kv_fill_fp8(const void* k, const void* v, long long tok_stride,
+                                     long long head_stride, const int32_t* cu_seqlens,
+                                     const int32_t* start_pos, const int32_t* seq_rows,
+                                     int n_seqs, int max_seqlen, int Hkv, int head_dim,
+                                     void* k_pool, void* v_pool, float* k_scale, float* v_scale,
+                                     const int32_t* block_tables, int page_table_rows,
+                                     int max_blocks_per_seq, int block_size, int num_blocks,
+                                     void* stream) {
+  return kv_fill_fp8(k, v, tok_stride, head_stride, cu_seqlens, start_pos, seq_rows, 0, n_seqs,
+                     max_seqlen, Hkv, head_dim, k_pool, v_pool, k_scale, v_scale, block_tables,
+                     page_table_rows, max_blocks_per_seq, block_size, num_blocks, stream);
+}
+
+extern "C" int sym_paged_kv_fill_fp8_packed(
+    const void* k, const void* v, const int32_t* cu_seqlens, const int32_t* positions,
+    const int32_t* seq_ids, int T, int n_seqs, int max_seqlen, int Hkv, int head_dim, void* k_pool,
+    void* v_pool, float* k_scale, float* v_scale, const int32_t* block_tables,
+    int page_table_rows, int max_blocks_per_seq, int block_size, int num_blocks, void* stream) {
+  SYM_REQUIRE(T >= 0, SYM_ERR_INVALID, "paged_kv_fill_fp8_packed: T=%d < 0", T);
+  if (T == 0) return SYM_OK;
+  SYM_REQUIRE(positions && seq_ids, SYM_ERR_INVALID,
+              "paged_kv_fill_fp8_packed: null pointer argument");
+  return kv_fill_fp8(k, v, (long long)Hkv * head_dim, head_dim, cu_seqlens, positions, seq_ids, T,
+                     n_seqs, max_seqlen, Hkv, head_dim, k_pool, v_pool, k_scale, v_scale,
+                     block_tables, page_table_rows, max_blocks_per_seq, block_size, num_blocks,
+                     stream);
 }

@@ -653,6 +653,36 @@ def paged_kv_fill_fp8(k: torch.Tensor, v: torch.Tensor, cu_seqlens: torch.Tensor
               lay.block_size, lay.num_blocks, _stream())
 
 
+def paged_kv_fill_fp8_packed(k: torch.Tensor, v: torch.Tensor, cu_seqlens: torch.Tensor,
+                             max_seqlen: int, positions: torch.Tensor, seq_ids: torch.Tensor,
+                             k_pool: torch.Tensor, v_pool: torch.Tensor, k_scale: torch.Tensor,
+                             v_scale: torch.Tensor, block_tables: torch.Tensor) -> None:
+    """:func:`paged_kv_fill_fp8` of packed tokens k, v [T, Hkv, D], each sequence starting at its
+    first token's position in its first token's page-table row (positions, seq_ids [T])."""
+    _check(k, "k", torch.bfloat16)
+    _check(v, "v", torch.bfloat16, k.device)
+    _check_shape(v, "v", tuple(k.shape))
+    if k.dim() != 3 or k.shape[2] != HEAD_DIM:
+        raise ValueError(f"k must be 3-D with head_dim {HEAD_DIM}, got {tuple(k.shape)}")
+    _check(cu_seqlens, "cu_seqlens", torch.int32, k.device)
+    n = cu_seqlens.numel() - 1
+    if n < 0 or cu_seqlens.dim() != 1:
+        raise ValueError("cu_seqlens must be [n_seqs + 1]")
+    lay = _check_pools(k_pool, v_pool, block_tables, 1, k_scale, v_scale)
+    if k_pool.dtype != torch.float8_e4m3fn:
+        raise TypeError("paged_kv_fill_fp8_packed needs float8_e4m3fn pools")
+    T, hkv, _ = k.shape
+    if hkv != lay.num_kv_heads:
+        raise ValueError(f"k has {hkv} kv heads, the pool {lay.num_kv_heads}")
+    for t, name in ((positions, "positions"), (seq_ids, "seq_ids")):
+        _check(t, name, torch.int32, k.device, align=4)
+        _check_shape(t, name, (T,))
+    _lib.call("sym_paged_kv_fill_fp8_packed", _ptr(k), _ptr(v), _ptr(cu_seqlens), _ptr(positions),
+              _ptr(seq_ids), T, n, int(max_seqlen), hkv, HEAD_DIM, _ptr(k_pool), _ptr(v_pool),
+              _ptr(k_scale), _ptr(v_scale), _ptr(block_tables), block_tables.shape[0],
+              lay.max_blocks_per_seq, lay.block_size, lay.num_blocks, _stream())
+
+
 # -------------------------------------------------------------------------------------------
 def embedding(ids: torch.Tensor, table: torch.Tensor,
               out: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -242,12 +242,10 @@ class HIPBailingMoEAttention(StatefulHIPModule):
             rotary_dim=self.rotary_dim, rope_cs=d["rope"], q_norm_w=d["q_norm"],
             k_norm_w=d["k_norm"], eps=self.norm_eps)
         if cache.is_fp8 and T > 0:
-            first = cu_seqlens[:-1].long().clamp(max=T - 1)
-            hip_ops.paged_kv_fill_fp8(
-                k, v, cu_seqlens, max_seqlen, cache.key_cache(self.layer_idx),
+            hip_ops.paged_kv_fill_fp8_packed(
+                k, v, cu_seqlens, max_seqlen, positions, seq_ids, cache.key_cache(self.layer_idx),
                 cache.value_cache(self.layer_idx), cache.key_scale(self.layer_idx),
-                cache.value_scale(self.layer_idx), cache.page_table_device,
-                start_pos=positions[first].contiguous(), seq_rows=seq_ids[first].contiguous())
+                cache.value_scale(self.layer_idx), cache.page_table_device)
         o = hip_ops.prefill_attention(q, k, v, cu_seqlens, max_seqlen, self.scaling)
         if residual is not None:
             return hip_ops.gemm(o.view(-1, self.num_heads * self.head_dim), d["dense_w"],
