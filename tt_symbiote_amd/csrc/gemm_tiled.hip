@@ -8,8 +8,7 @@
 // Design (gfx950). What bounds these kernels was measured, not assumed: a wave-wide load of
 // 16 rows x 64 bytes (a 32-column step of K-major rows) reaches ~30 B/clk per CU from L2, one of
 // 8 rows x 128 bytes ~50 B/clk, while LDS reads (~190 B/clk) and back-to-back MFMAs (94% of
-// peak) have room; and the chip clocks down to 2.0-2.25 GHz under these kernels. Two tile
-// shapes (and a thin variant of the first):
+// peak) have room; and the chip clocks down to 2.0-2.25 GHz under these kernels. The tiles:
 //   gemm_tile_kernel / gemm_tile_persistent (dense projections; grouped gate/up and down on a
 //     persistent grid while the segment list has at most 512 entries): 256 x 256 tiles, one
 //     workgroup of 8 waves per CU, each wave a 64 x 128 block (4 x 8 v_mfma_f32_16x16x32_bf16
@@ -18,11 +17,14 @@
 //     overlap the other half's MFMAs, with one barrier per step. In the persistent kernels a
 //     tile of at most 64 valid rows runs thin_tile instead: three 40 KB stages (64 A rows and
 //     256 B rows each), two steps of lookahead.
-//   gemm_small_kernel: 32 x 64 to 128 x 256 tiles for dense GEMMs of few rows (dense_tiling).
-//   gemm_tile128_kernel (grouped down projection over longer segment lists): 128 x 256 tiles, two workgroups of 8 waves per CU, each
-//     wave a 64 x 64 block; 32 columns per step through a 3-stage 72 KB ring. The second
-//     workgroup covers a tile's prologue (segment lookup, first loads) and epilogue, which a
-//     one-workgroup shape leaves bare at 16 steps.
+//   gemm_small_kernel: 32 x 64 to 128 x 256 tiles for dense GEMMs of few rows (dense_tiling), with
+//     long K split over several workgroups (dense_splits); gemm_narrow_persistent: 64 x 128 tiles
+//     of the grouped products while experts have few rows each (narrow_tiles).
+//   gemm_f8_persistent: 128 x 256 tiles over fp8 expert weights, converted in registers.
+//   gemm_tile128_kernel (grouped down projection over segment lists of more than 512 entries):
+//     128 x 256 tiles, two workgroups of 8 waves per CU, each wave a 64 x 64 block; 32 columns per
+//     step through a 3-stage 72 KB ring. The second workgroup covers a tile's prologue (segment
+//     lookup, first loads) and epilogue, which a one-workgroup shape leaves bare at 16 steps.
 // Operand tiles go from global memory straight into LDS (global_load_lds_dwordx4, no register
 // staging). A wave-wide LDS-DMA instruction writes 1 KB contiguously: lane l takes row l / c,
 // 16-byte slot l % c (c = chunks per row), fetching global chunk (l % c) ^ swz(row), so that

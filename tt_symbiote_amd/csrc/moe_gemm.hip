@@ -760,14 +760,15 @@ __global__ __launch_bounds__(kGemmThreads) void moe_gate_up_tok_kernel(
     const uint8_t* wg = (const uint8_t*)w_gu + ((size_t)m.e * 2 * I + col0 + r16) * (size_t)H + kq * 32;
     const float* sg = s_gu + ((size_t)m.e * ((2 * I) >> 7) + (col0 >> 7)) * nsteps;
     const float* su = s_gu + ((size_t)m.e * ((2 * I) >> 7) + ((I + col0) >> 7)) * nsteps;
-    gate_up_pass_fp8<U, true>(x, H, nullptr, m.t, wg, wg + (size_t)I * H, sg, su, s_beg, s_end, r16, kq, accg[0],
-                        accu[0]);
+    gate_up_pass_fp8<U, true>(x, H, nullptr, m.t, wg, wg + (size_t)I * H, sg, su, s_beg, s_end, r16,
+                              kq, accg[0], accu[0]);
   } else {
     const int nsteps = H >> 6;
     const int s_beg = (wave * nsteps) >> 2, s_end = ((wave + 1) * nsteps) >> 2;
     const uint16_t* wg =
         (const uint16_t*)w_gu + ((size_t)m.e * 2 * I + col0 + r16) * (size_t)H + kq * kKLane;
-    gate_up_pass<U, true>(x, H, nullptr, m.t, wg, wg + (size_t)I * H, s_beg, s_end, r16, kq, accg[0], accu[0]);
+    gate_up_pass<U, true>(x, H, nullptr, m.t, wg, wg + (size_t)I * H, s_beg, s_end, r16, kq, accg[0],
+                          accu[0]);
   }
   gate_up_epilogue<1>(s_red, accg, accu, wave, lane, 1, (size_t)a, I, col0, h);
 }

@@ -190,10 +190,11 @@ __global__ __launch_bounds__(256) void attn_decode_prologue_kernel(
 
 // The same for many tokens (prefill), bit for bit: a wave takes one token, 16 lanes a head (8
 // consecutive dims = 16 bytes per lane), so a token's Hq + 2 Hkv heads are a few 1 KB loads issued
-// together instead of two 2-byte loads per lane and head one after another. Bound by memory (qkv in,
-// q, k, v and the pool slots out: 133 MB at 9322 tokens with Hq = 16, Hkv = 4, 40 -> 34 us). The sum of squares is the wave sum's tree: dims d and d + 64 first, then partners 32, 16, 8
-// apart (lane rotations by 8, 4, 2, 1 in a row of 16: after each step the values repeat with
-// that period) and 4, 2, 1 apart (within the lane). RoPE's pairs are rd / 2 dims apart, i.e. rd / 16
+// together instead of two 2-byte loads per lane and head one after another. Bound by memory (qkv
+// in, q, k, v and the pool slots out: 133 MB at 9322 tokens with Hq = 16, Hkv = 4, 40 -> 34 us). The
+// sum of squares is the wave sum's tree: dims d and d + 64 first, then partners 32, 16, 8 apart
+// (lane rotations by 8, 4, 2, 1 in a row of 16: after each step the values repeat with that
+// period) and 4, 2, 1 apart (within the lane). RoPE's pairs are rd / 2 dims apart, i.e. rd / 16
 // lanes: rd % 16 == 0.
 constexpr int kPrologueHeads = 6;  // heads per 16-lane group in flight
 
