@@ -435,6 +435,20 @@ def test_grouped_tiled_row_rule(device, T, E, H, I, top_k):
                                    atol=1e-4)
 
 
+@pytest.mark.parametrize("T,H,y_dtype,kernel", [
+    (191, 256, torch.float32, "stream"), (192, 256, torch.float32, "tiled"),
+    # sizes and outputs that only the tiled kernels take: from 128 tokens, as before
+    (128, 256, torch.bfloat16, "tiled"), (150, 320, torch.float32, "tiled"),
+])
+def test_grouped_auto_rule(device, T, H, y_dtype, kernel):
+    """kernel="auto" gives the bits of the kernels its rule names."""
+    x, wgu, wd, res = _gemm_case(T, 64, H, 128, 6, seed=T, device=device, skew=False)
+    x, wgu, wd = x.to(device), wgu.to(device), wd.to(device)
+    got = hip_ops.moe_grouped_swiglu(x, res, wgu, wd, y_dtype=y_dtype)
+    want = hip_ops.moe_grouped_swiglu(x, res, wgu, wd, y_dtype=y_dtype, kernel=kernel)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_grouped_tiled_workspace_reentrant(device):
     """The tiled grouped GEMMs keep their tile counters in the caller's workspace: two streams
     running prefill-size launches at the same time, each with its own workspace, give the bytes

@@ -908,7 +908,13 @@ def moe_route_permute(logits: torch.Tensor, bias: torch.Tensor, *, n_group: int,
     return res
 
 
-TILED_MIN_TOKENS = 128  # from this many tokens the expert GEMMs use the tiled (MFMA-bound) kernels
+# From this many tokens the expert GEMMs use the tiled (MFMA-bound) kernels (gate/up + down of 257
+# segments of 512 x 2048, us, streaming against tiled, even / Zipf load: 128 tokens 260 / 222 against
+# 294 / 251, 160: 266 / 239 against 310 / 269, 192: 269 / 286 against 314 / 281, 256: 280 / 316
+# against 315 / 291).
+TILED_MIN_TOKENS = 192
+# From this many where the streaming kernels do not apply (H % 256 != 0, bf16 y).
+TILED_ONLY_MIN_TOKENS = 128
 
 # The same for fp8 expert weights, gate/up and down apart: the streaming down kernel keeps its
 # weights in registers for all 16-row passes, the gate/up kernel re-reads them. 257 segments of 512
@@ -977,12 +983,13 @@ def moe_grouped_swiglu(x: torch.Tensor, route: RouteResult, w_gate_up,
     """h = silu(x Wg^T) * (x Wu^T), y = h Wd^T per segment; returns (h [rows, I], y [rows, H]).
     The weights are bf16 tensors, or BlockFp8 (fp8 e4m3fn + 128 x 128 block scales, dequantized
     in the kernel). ``kernel``: "stream" (weight-streaming kernels for decode-size segments),
-    "tiled" (256 x 256 / 128 x 256 MFMA tiles for prefill-size segments, bf16 only) or "auto"
-    (tiled from TILED_MIN_TOKENS tokens with bf16 weights). ``y_dtype``: fp32, or bf16 with the tiled kernels
-    (half the bytes of y written and read back by the combine). ``workspace``: the tiled
-    kernels' tile counters (:func:`moe_tiled_workspace`, zeroed, left zeroed by every launch);
-    a fresh one per call when None. Calls that may overlap on different streams need different
-    workspaces."""
+    "tiled" (MFMA tiles for prefill-size segments, bf16 weights only) or "auto" (tiled from
+    TILED_MIN_TOKENS tokens, or TILED_ONLY_MIN_TOKENS where only the tiled kernels apply; fp8
+    weights: from TILED_MIN_TOKENS_FP8 / TILED_MIN_TOKENS_FP8_DOWN). ``y_dtype``: fp32, or bf16
+    with the tiled bf16 kernels (half the bytes of y written and read back by the combine).
+    ``workspace``: the tiled bf16 kernels' tile counters (:func:`moe_tiled_workspace`, zeroed, left
+    zeroed by every launch); a fresh one per call when None. Calls that may overlap on different
+    streams need different workspaces."""
     _check(x, "x", torch.bfloat16)
     if x.dim() != 2:
         raise ValueError(f"x must be [T, H], got {tuple(x.shape)}")
@@ -1016,7 +1023,9 @@ def moe_grouped_swiglu(x: torch.Tensor, route: RouteResult, w_gate_up,
         h = torch.empty(rows, I, dtype=torch.bfloat16, device=dev)
     if kernel not in ("auto", "stream", "tiled"):
         raise ValueError(f"kernel {kernel!r}")
-    tiled = not fp8 and (kernel == "tiled" or (kernel == "auto" and T >= TILED_MIN_TOKENS))
+    only = H % 256 != 0 or y_dtype == torch.bfloat16
+    tiled = not fp8 and (kernel == "tiled" or (kernel == "auto" and T >= (
+        TILED_ONLY_MIN_TOKENS if only else TILED_MIN_TOKENS)))
     if y_dtype not in (torch.float32, torch.bfloat16):
         raise TypeError(f"y_dtype {y_dtype} (fp32 or bf16)")
     if y_dtype == torch.bfloat16 and not tiled:
